@@ -122,20 +122,52 @@ __global__ void __launch_bounds__(kReduceBlock) k_wl_finalize(const double2* par
     if (threadIdx.x == 0) out[T] = make_double2(acc.x * scale, acc.y * scale);
 }
 
-__global__ void __launch_bounds__(kReduceBlock) k_wlop_finalize(const double* partials, int nb, double* accum) {
-    const double* p = partials + (size_t)blockIdx.x * nb;
-    double acc = 0.0;
-    int i = threadIdx.x;
-    for (; i + (kSumBatch - 1) * kReduceBlock < nb; i += kSumBatch * kReduceBlock) {
-        double v[kSumBatch];
+// 64 outputs per workgroup.  Matrix-core partials [rows][T][i][j]: wave w adds rows
+// w, w + 4, ... of its lane's output, then the four waves in order.  Partials of the
+// fallback [(i nop + j) T1 + T][nb]: wave w takes the outputs w, w + 4, ... with its lanes
+// over nb.
+__global__ void __launch_bounds__(kReduceBlock) k_wlop_finalize(const double* partials, int rows, int nb, int nop,
+                                                                int T1, const int* state, int nstate, double* accum) {
+    __shared__ double ws[kReduceBlock / 64][64];
+    int any = 0;
+    for (int i = threadIdx.x; i < nstate; i += kReduceBlock) any |= state[i] == kLinesBad;
+    any = __syncthreads_or(any);
+    const int nout = nop * nop * T1, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    constexpr int kW = kReduceBlock / 64;
+    if (any) {
+        for (int k = w; k < 64; k += kW) {
+            const int o = blockIdx.x * 64 + k;
+            if (o >= nout) break;
+            double acc = 0.0;
+            for (int i = lane; i < nb; i += 64) acc += partials[(size_t)o * nb + i];
 #pragma unroll
-        for (int k = 0; k < kSumBatch; k++) v[k] = p[i + k * kReduceBlock];
-#pragma unroll
-        for (int k = 0; k < kSumBatch; k++) acc += v[k];
+            for (int off = 32; off > 0; off >>= 1) acc += __shfl_down(acc, off, 64);
+            if (lane == 0) accum[o] += acc;
+        }
+        return;
     }
-    for (; i < nb; i += kReduceBlock) acc += p[i];
-    const double2 v = block_sum_all(make_double2(acc, 0.0));
-    if (threadIdx.x == 0) accum[blockIdx.x] += v.x;
+    const int o = blockIdx.x * 64 + lane;
+    double acc = 0.0;
+    if (o < nout) {
+        int i = w;
+        for (; i + (kSumBatch - 1) * kW < rows; i += kSumBatch * kW) {
+            double v[kSumBatch];
+#pragma unroll
+            for (int k = 0; k < kSumBatch; k++) v[k] = partials[(size_t)(i + k * kW) * nout + o];
+#pragma unroll
+            for (int k = 0; k < kSumBatch; k++) acc += v[k];
+        }
+        for (; i < rows; i += kW) acc += partials[(size_t)i * nout + o];
+    }
+    ws[w][lane] = acc;
+    __syncthreads();
+    if (w == 0 && o < nout) {
+        acc = ws[0][lane];
+#pragma unroll
+        for (int k = 1; k < kW; k++) acc += ws[k][lane];
+        const int T = o / (nop * nop), ij = o - T * nop * nop;
+        accum[(size_t)ij * T1 + T] += acc;
+    }
 }
 
 __global__ void __launch_bounds__(kReduceBlock) k_batch_finalize(const BatchEntry* table, double2* out) {
@@ -236,9 +268,12 @@ hipError_t launch_wl_finalize(const double2* partials, int nb, int tmax, double 
     return hipGetLastError();
 }
 
-hipError_t launch_wlop_finalize(const double* partials, int nb, int nout, double* accum, hipStream_t s) {
+hipError_t launch_wlop_finalize(const double* partials, int rows, int nb, int nop, int T1, const int* state,
+                                int nstate, double* accum, hipStream_t s) {
+    const int nout = nop * nop * T1;
     if (nout <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_wlop_finalize, dim3(nout), dim3(kReduceBlock), 0, s, partials, nb, accum);
+    hipLaunchKernelGGL(k_wlop_finalize, dim3((nout + 63) / 64), dim3(kReduceBlock), 0, s, partials, rows, nb, nop, T1,
+                       state, nstate, accum);
     return hipGetLastError();
 }
 

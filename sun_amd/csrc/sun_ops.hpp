@@ -181,13 +181,20 @@ struct OpsTable {
     hipError_t (*wl_loops)(const Field& f, const Field& lines, const Geom&, int r, int tmax, double2* partials,
                            hipStream_t);
     // operator-basis Wilson loops: the operator fields of direction mu at radius r
-    // (family 0: 10 slots, 1: 25; V 18-real entries per slot, slot k at k * stride
-    // bytes after ops0 in every plane; rt8 = 2 sqrt 2), and the correlator of every
-    // slot pair, nop^2 (tmax + 1) * monitor_blocks(geom) FP64 partials
-    hipError_t (*wlop_fields)(const Field& f, const Field& ops0, size_t stride, const Geom&, int family, int r,
+    // (family 0: 10 slots, 1: 25; slot k, V matrices of 2 N^2 reals one after another, at
+    // ops + k * stride; rt8 = 2 sqrt 2)
+    hipError_t (*wlop_fields)(const Field& f, char* ops, size_t stride, const Geom&, int family, int r,
                               int mu, double rt8, hipStream_t);
-    hipError_t (*wlop_corr)(const Field& f, const Field& ops0, size_t stride, const Geom&, int nop, int r, int mu,
-                            int tmax, double* partials, hipStream_t);
+    // time lines of every spatial site: P of `next` times, inverses Q (may be null) of X3
+    // times, FP64 N x N matrices; state[line_blocks(geom)]: per block whether its lines are
+    // unitary (0), have condition numbers up to cond (1) or not (kLinesBad)
+    hipError_t (*time_lines)(const Field& f, const Geom&, int next, double cond, double* P, double* Q, int* state,
+                             hipStream_t);
+    // the correlator of every slot pair; time lines of next = X3 + tmax times.  Partials:
+    // [wlop_corr_blocks][T][i][j], or, where a state is kLinesBad,
+    // [(i nop + j)(tmax + 1) + T][monitor_blocks]
+    hipError_t (*wlop_corr)(const Field& f, char* ops, size_t stride, const Geom&, int nop, int r, int mu,
+                            int tmax, const double* P, const double* Q, const int* state, double* partials, hipStream_t);
     int max_block;   // largest workgroup the update kernels are compiled for
     int has_piped;   // the variant has the software-pipelined overrelaxation kernel
     int piped_max_block;
@@ -246,6 +253,13 @@ inline int partial_slots(const Geom& g) {
     const int a = 3 * monitor_blocks(g), b = plaquette_blocks(g) + polyakov_blocks(g);
     return a > b ? a : b;
 }
+// state of time lines that the measurement kernels cannot invert
+constexpr int kLinesBad = 2;
+// workgroups of the time-line kernel (64 spatial sites each)
+inline int line_blocks(const Geom& g) { return (g.str[3] + 63) / 64; }
+// workgroups of the matrix-core correlator, one per CU (its LDS), each with an equal share
+// of the spatial sites
+inline int wlop_corr_blocks(const Geom& g) { return g.str[3] < 256 ? g.str[3] : 256; }
 inline int update_blocks(const Geom& g, int block) { return (g.half + block - 1) / block; }
 inline int link_blocks(const Geom& g) { return (4 * g.V + kReduceBlock - 1) / kReduceBlock; }
 
@@ -260,8 +274,10 @@ hipError_t launch_finalize_iteration(const double2* partials, int pb, int qb, do
 // Wilson loops of one radius: out[T] = scale * sum over mu < 3 and the nb partials
 // of (mu, T), T = 0..tmax, in a fixed order
 hipError_t launch_wl_finalize(const double2* partials, int nb, int tmax, double scale, double2* out, hipStream_t s);
-// accum[o] += the sum of partials[o nb .. o nb + nb) in a fixed order, o < nout
-hipError_t launch_wlop_finalize(const double* partials, int nb, int nout, double* accum, hipStream_t s);
+// accum[(i nop + j) T1 + T] += the sum of the correlator's partials in a fixed order:
+// [rows][T][i][j], or [(i nop + j) T1 + T][nb] where one of the nstate states is kLinesBad
+hipError_t launch_wlop_finalize(const double* partials, int rows, int nb, int nop, int T1, const int* state,
+                                int nstate, double* accum, hipStream_t s);
 // link monitor: out[0] = trace sum * scale_tr, out[1] = determinant sum * scale_det,
 // out[2] = (max deviation, max |det - 1|) from the three segments of n partials
 hipError_t launch_monitor_finalize(const double2* partials, int n, double scale_tr, double scale_det, double2* out,

@@ -8,6 +8,7 @@
 // varies); here every (pair, T) is a fixed-order sum of per-workgroup partials.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <vector>
@@ -23,7 +24,10 @@ struct sun_wlop {
     size_t stride = 0;      // bytes of one slot (V entries)
     void* ops = nullptr;    // nop slots
     double* partials = nullptr;
-    int nb = 0;
+    int nb = 0, rows = 0;   // workgroups of the fallback and of the matrix-core correlator
+    double* lines = nullptr;   // time lines: X3 + tmax times of every spatial site
+    double* inverses = nullptr;  // their inverses, X3 times
+    int* state = nullptr;   // per block of lines, whether they are unitary or can be inverted
     double* acc = nullptr;  // nop^2 (tmax + 1), (i nop + j)(tmax + 1) + T
     int r = -1, mu = -1;    // radius and direction of the current operator field
 };
@@ -36,6 +40,9 @@ void release(sun_wlop* h) {
     if (!h) return;
     if (h->ops) hipFree(h->ops);
     if (h->partials) hipFree(h->partials);
+    if (h->lines) hipFree(h->lines);
+    if (h->inverses) hipFree(h->inverses);
+    if (h->state) hipFree(h->state);
     if (h->acc) hipFree(h->acc);
     delete h;
 }
@@ -67,10 +74,16 @@ extern "C" int sun_wlop_create(sun_lattice* lat, int family, int tmax, sun_wlop*
     h->tmax = tmax;
     h->lb = (size_t)2 * lat->d.nc * lat->d.nc * (size_t)lat->d.precision;
     h->stride = (size_t)g.V * h->lb;
-    h->nb = monitor_blocks(g);  // the correlator's 256-site blocks
+    h->nb = monitor_blocks(g);
+    h->rows = wlop_corr_blocks(g);
     const size_t nout = (size_t)nop * nop * (tmax + 1);
     HIP_TRY_CLEANUP(hipMalloc(&h->ops, (size_t)nop * h->stride), release(h));
-    HIP_TRY_CLEANUP(hipMalloc((void**)&h->partials, nout * h->nb * sizeof(double)), release(h));
+    const size_t npart = nout * (size_t)std::max(h->nb, h->rows);
+    const size_t line = (size_t)2 * lat->d.nc * lat->d.nc * sizeof(double), vs = (size_t)g.str[3];
+    HIP_TRY_CLEANUP(hipMalloc((void**)&h->partials, npart * sizeof(double)), release(h));
+    HIP_TRY_CLEANUP(hipMalloc((void**)&h->lines, vs * (g.X[3] + tmax) * line), release(h));
+    HIP_TRY_CLEANUP(hipMalloc((void**)&h->inverses, vs * g.X[3] * line), release(h));
+    HIP_TRY_CLEANUP(hipMalloc((void**)&h->state, line_blocks(g) * sizeof(int)), release(h));
     HIP_TRY_CLEANUP(hipMalloc((void**)&h->acc, nout * sizeof(double)), release(h));
     HIP_TRY_CLEANUP(hipMemset(h->acc, 0, nout * sizeof(double)), release(h));
     *out = h;
@@ -93,10 +106,30 @@ extern "C" int sun_wlop_fields(sun_wlop* h, int r, int mu, void* stream) {
     sun_lattice* lat = h->lat;
     hipStream_t s = pick_stream(lat, stream);
     HIP_TRY(hipSetDevice(lat->ctx->device));
-    const Field ops0 = make_field(h->ops, (size_t)lat->g.V, h->lb);
-    HIP_TRY(lat->ops->wlop_fields(lat->f, ops0, h->stride, lat->g, h->family, r, mu, 2.0 * std::sqrt(2.0), s));
+    HIP_TRY(lat->ops->wlop_fields(lat->f, (char*)h->ops, h->stride, lat->g, h->family, r, mu, 2.0 * std::sqrt(2.0), s));
     h->r = r;
     h->mu = mu;
+    return SUN_OK;
+}
+
+// Condition number up to which time lines are inverted, FP32 and FP64 lattices (whose X and
+// Y are formed in FP32 and FP64): rounding errors grow by at most its square, to about 1e-12
+// of a loop in FP64 and, in FP32, to what a dozen products of FP32 links carry.
+constexpr double kLineCond[2] = {4.0, 100.0};
+
+// the time lines of the lattice's present temporal links
+static int time_lines(sun_wlop* h, hipStream_t s) {
+    HIP_TRY(h->lat->ops->time_lines(h->lat->f, h->lat->g, h->lat->g.X[3] + h->tmax, kLineCond[h->lat->d.precision == SUN_PREC_F64], h->lines, h->inverses, h->state, s));
+    return SUN_OK;
+}
+
+// the correlators of the current operator field, the time lines being there
+static int correlate(sun_wlop* h, int r, int mu, hipStream_t s) {
+    sun_lattice* lat = h->lat;
+    HIP_TRY(lat->ops->wlop_corr(lat->f, (char*)h->ops, h->stride, lat->g, h->nop, r, mu, h->tmax, h->lines, h->inverses, h->state,
+                                h->partials, s));
+    HIP_TRY(launch_wlop_finalize(h->partials, h->rows, h->nb, h->nop, h->tmax + 1, h->state, line_blocks(lat->g), h->acc,
+                                 s));
     return SUN_OK;
 }
 
@@ -107,10 +140,8 @@ extern "C" int sun_wlop_correlate(sun_wlop* h, int r, int mu, void* stream) {
     sun_lattice* lat = h->lat;
     hipStream_t s = pick_stream(lat, stream);
     HIP_TRY(hipSetDevice(lat->ctx->device));
-    const Field ops0 = make_field(h->ops, (size_t)lat->g.V, h->lb);
-    HIP_TRY(lat->ops->wlop_corr(lat->f, ops0, h->stride, lat->g, h->nop, r, mu, h->tmax, h->partials, s));
-    HIP_TRY(launch_wlop_finalize(h->partials, h->nb, h->nop * h->nop * (h->tmax + 1), h->acc, s));
-    return SUN_OK;
+    SUN_TRY(time_lines(h, s));
+    return correlate(h, r, mu, s);
 }
 
 extern "C" int sun_wlop_clear(sun_wlop* h, void* stream) {
@@ -165,28 +196,18 @@ static int sun_wlop_fields_to_host_body(sun_wlop* h, double* out) {
     HIP_TRY(hipSetDevice(lat->ctx->device));
     HIP_TRY(hipStreamSynchronize(pick_stream(lat, nullptr)));
     HIP_TRY(hipDeviceSynchronize());
-    const size_t V = (size_t)lat->g.V, lb = h->lb;
+    const size_t V = (size_t)lat->g.V;
     const int nreal = 2 * lat->d.nc * lat->d.nc;
     const bool f32 = lat->d.precision == SUN_PREC_F32;
-    const size_t nfull = lb / 16, tail = lb % 16;
-    std::vector<unsigned char> raw(h->stride);
+    std::vector<float> raw(f32 ? V * nreal : 0);
     for (int k = 0; k < h->nop; k++) {
-        HIP_TRY(hipMemcpy(raw.data(), (char*)h->ops + (size_t)k * h->stride, h->stride, hipMemcpyDeviceToHost));
-        for (size_t l = 0; l < V; l++) {
-            unsigned char rec[16 * kMaxPlanes];
-            for (size_t c = 0; c < nfull; c++) memcpy(rec + 16 * c, raw.data() + c * V * 16 + l * 16, 16);
-            if (tail) memcpy(rec + 16 * nfull, raw.data() + nfull * V * 16 + l * 8, 8);
-            double* dst = out + ((size_t)k * V + l) * nreal;
-            for (int q = 0; q < nreal; q++) {
-                if (f32) {
-                    float v;
-                    memcpy(&v, rec + 4 * q, 4);
-                    dst[q] = v;
-                } else {
-                    memcpy(dst + q, rec + 8 * q, 8);
-                }
-            }
+        double* dst = out + (size_t)k * V * nreal;
+        if (!f32) {
+            HIP_TRY(hipMemcpy(dst, (char*)h->ops + (size_t)k * h->stride, h->stride, hipMemcpyDeviceToHost));
+            continue;
         }
+        HIP_TRY(hipMemcpy(raw.data(), (char*)h->ops + (size_t)k * h->stride, h->stride, hipMemcpyDeviceToHost));
+        for (size_t q = 0; q < V * nreal; q++) dst[q] = raw[q];
     }
     return SUN_OK;
 }
@@ -206,12 +227,13 @@ static int sun_wilson_loops_ops_body(sun_lattice* lat, int family, int rmax, int
     SUN_TRY(sun_wlop_create(lat, family, tmax, &h));
     const size_t n = (size_t)h->nop * h->nop * (tmax + 1);
     const double norm = (double)g.V * 3.0 * lat->d.nc;  // test.cpp:290
-    int rc = SUN_OK;
+    const hipStream_t s = pick_stream(lat, stream);
+    int rc = time_lines(h, s);
     for (int r = 2; r <= rmax && rc == SUN_OK; r++) {
         rc = sun_wlop_clear(h, stream);
         for (int mu = 0; mu < 3 && rc == SUN_OK; mu++) {
             rc = sun_wlop_fields(h, r, mu, stream);
-            if (rc == SUN_OK) rc = sun_wlop_correlate(h, r, mu, stream);
+            if (rc == SUN_OK) rc = correlate(h, r, mu, s);
         }
         if (rc == SUN_OK) rc = sun_wlop_read(h, out + (size_t)(r - 2) * n, stream);
         if (rc == SUN_OK)
