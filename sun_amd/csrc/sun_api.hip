@@ -44,7 +44,7 @@ extern "C" const char* sun_version(void) { return "sun-mi355x 0.1 (gfx950)"; }
 // under stream capture, serving loops).  In host code `scratch` names a host-side
 // stand-in, not device memory: its device address on each GPU is looked up once, at
 // the first sun_init on that device, and only that address is used afterwards.
-static __device__ __align__(256) unsigned char scratch[sun::kNoAllocScratchBytes];
+static __device__ __align__(256) unsigned char scratch[sun::kNoAllocScratchBytes + sun::kNoAllocStateBytes];
 
 namespace {
 constexpr int kMaxDevices = 64;

@@ -109,17 +109,47 @@ __global__ void __launch_bounds__(kReduceBlock) k_finalize_iteration(const doubl
     }
 }
 
-__global__ void __launch_bounds__(kReduceBlock) k_wl_finalize(const double2* partials, int nb, int tmax, double scale,
-                                                              double2* out) {
+__global__ void __launch_bounds__(kReduceBlock) k_wl_finalize(const double2* partials, int nb_unitary, int nb_general,
+                                                              int nb_bad, int tmax, double scale, const int* state,
+                                                              int nstate, double2* out) {
+    int nb = nb_bad;
+    if (state) {
+        int bad = 0, general = 0;
+        for (int i = threadIdx.x; i < nstate; i += kReduceBlock) {
+            bad |= state[i] == kLinesBad;
+            general |= state[i] != 0;
+        }
+        bad = __syncthreads_or(bad);
+        general = __syncthreads_or(general);
+        nb = bad ? nb_bad : general ? nb_general : nb_unitary;
+    }
+    if (!nb) return;
     const int T = blockIdx.x;
     double2 acc = make_double2(0.0, 0.0);
     for (int mu = 0; mu < 3; mu++) {
-        const double2 v = ordered_sum(partials + (size_t)(mu * (tmax + 1) + T) * nb, nb);
+        const double2 v = ordered_sum(partials + (size_t)((blockIdx.y * 3 + mu) * (tmax + 1) + T) * nb, nb);
         __syncthreads();
         acc.x += v.x;
         acc.y += v.y;
     }
-    if (threadIdx.x == 0) out[T] = make_double2(acc.x * scale, acc.y * scale);
+    if (threadIdx.x == 0) out[blockIdx.y * (tmax + 1) + T] = make_double2(acc.x * scale, acc.y * scale);
+}
+
+// partials [(i nop + j) T1 + T][nb], a workgroup per output
+__global__ void __launch_bounds__(kReduceBlock) k_wlop_finalize_direct(const double* partials, int nb, double* accum) {
+    const double* p = partials + (size_t)blockIdx.x * nb;
+    double acc = 0.0;
+    int i = threadIdx.x;
+    for (; i + (kSumBatch - 1) * kReduceBlock < nb; i += kSumBatch * kReduceBlock) {
+        double v[kSumBatch];
+#pragma unroll
+        for (int k = 0; k < kSumBatch; k++) v[k] = p[i + k * kReduceBlock];
+#pragma unroll
+        for (int k = 0; k < kSumBatch; k++) acc += v[k];
+    }
+    for (; i < nb; i += kReduceBlock) acc += p[i];
+    const double2 v = block_sum_all(make_double2(acc, 0.0));
+    if (threadIdx.x == 0) accum[blockIdx.x] += v.x;
 }
 
 // 64 outputs per workgroup.  Matrix-core partials [rows][T][i][j]: wave w adds rows
@@ -263,8 +293,10 @@ hipError_t launch_finalize_iteration(const double2* partials, int pb, int qb, do
     return hipGetLastError();
 }
 
-hipError_t launch_wl_finalize(const double2* partials, int nb, int tmax, double scale, double2* out, hipStream_t s) {
-    hipLaunchKernelGGL(k_wl_finalize, dim3(tmax + 1), dim3(kReduceBlock), 0, s, partials, nb, tmax, scale, out);
+hipError_t launch_wl_finalize(const double2* partials, const int nb[3], int nr, int tmax, double scale,
+                              const int* state, int nstate, double2* out, hipStream_t s) {
+    hipLaunchKernelGGL(k_wl_finalize, dim3(tmax + 1, nr), dim3(kReduceBlock), 0, s, partials, nb[0], nb[1], nb[2], tmax,
+                       scale, state, nstate, out);
     return hipGetLastError();
 }
 
@@ -272,7 +304,10 @@ hipError_t launch_wlop_finalize(const double* partials, int rows, int nb, int no
                                 int nstate, double* accum, hipStream_t s) {
     const int nout = nop * nop * T1;
     if (nout <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_wlop_finalize, dim3((nout + 63) / 64), dim3(kReduceBlock), 0, s, partials, rows, nb, nop, T1,
+    if (!state)
+        hipLaunchKernelGGL(k_wlop_finalize_direct, dim3(nout), dim3(kReduceBlock), 0, s, partials, nb, accum);
+    else
+        hipLaunchKernelGGL(k_wlop_finalize, dim3((nout + 63) / 64), dim3(kReduceBlock), 0, s, partials, rows, nb, nop, T1,
                        state, nstate, accum);
     return hipGetLastError();
 }

@@ -98,9 +98,11 @@ struct sun_ctx {
 
 namespace sun {
 // size of the device scratch array of the allocation-free entry points (one per
-// device, held until the process ends): sun_wilson_loops_noalloc keeps its Wilson-line
-// field (3V links in 18-real storage) and its partial sums there
+// device, held until the process ends): sun_wilson_loops_noalloc keeps its time lines or
+// its Wilson-line field (3V links in 18-real storage) and its partial sums there; behind
+// them the states of the time lines (at most 2731 blocks fit the rest)
 constexpr size_t kNoAllocScratchBytes = size_t(32) << 20;
+constexpr size_t kNoAllocStateBytes = size_t(16) << 10;
 // device result slots of a lattice: plaquette and Polyakov of sun_generate, or the
 // three of the link monitor
 constexpr int kResSlots = 3;

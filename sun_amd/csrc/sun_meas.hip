@@ -8,6 +8,7 @@
 // of the generation loop.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <vector>
 
 #include "sun_internal.hpp"
@@ -169,6 +170,65 @@ extern "C" int sun_multihit_ext(sun_lattice* in, sun_lattice* out, uint64_t seed
     return SUN_OK;
 }
 
+// Wilson loops by planes (sun_ops.hpp PlaneShape): the time lines, then radii in groups
+// whose partial sums fit what there is
+namespace {
+
+struct WlPlanes {
+    PlaneShape ps[2];        // unitary time lines, others
+    size_t lines, per_radius;  // bytes
+    bool fits() const { return ps[0].sites && ps[1].sites; }
+};
+
+WlPlanes wl_planes(const sun_lattice* lat, int tmax) {
+    const Geom& g = lat->g;
+    const size_t reals = (size_t)2 * lat->d.nc * lat->d.nc;
+    WlPlanes w;
+    w.ps[0] = plane_shape(g, tmax + 1, (int)(reals * lat->d.precision));
+    w.ps[1] = plane_shape(g, tmax + 1, (int)(reals * sizeof(double)));
+    w.lines = ((size_t)g.str[3] * (g.X[3] + 1) * reals * sizeof(double) + 255) & ~(size_t)255;
+    w.per_radius = (size_t)3 * (tmax + 1) * std::max(w.ps[0].blocks, w.ps[1].blocks) * sizeof(double2);
+    return w;
+}
+
+double wl_scale(const sun_lattice* lat) { return 1.0 / (3.0 * lat->d.nc * (double)lat->g.V); }  // wilsonloop.cu:512
+
+// Condition number up to which time lines are inverted (FP64 arithmetic), FP32 and FP64
+// lattices: rounding errors grow by at most its square
+constexpr double kWlCond[2] = {1e3, 1e2};
+
+int wl_by_planes(sun_lattice* lat, const WlPlanes& w, int rmax, int tmax, double* P, double2* part, size_t part_bytes,
+                 int* state, double2* res, hipStream_t s) {
+    const Geom& g = lat->g;
+    HIP_TRY(lat->ops->time_lines(lat->f, g, g.X[3] + 1, true, kWlCond[lat->d.precision == SUN_PREC_F64], P, nullptr,
+                                 state, s));
+    const int group = (int)std::min<size_t>((size_t)rmax + 1, part_bytes / w.per_radius);
+    const int nb[3] = {w.ps[0].blocks, w.ps[1].blocks, 0};
+    for (int r = 0; r <= rmax; r += group) {
+        const int hi = std::min(rmax + 1, r + group);
+        HIP_TRY(lat->ops->wl_plane(lat->f, g, r, hi, tmax + 1, g.X[3] + 1, P, state, w.ps, part, s));
+        HIP_TRY(launch_wl_finalize(part, nb, hi - r, tmax, wl_scale(lat), state, line_blocks(g),
+                                   res + (size_t)r * (tmax + 1), s));
+    }
+    return SUN_OK;
+}
+
+// every product multiplied out; where state is given, only if it is kLinesBad
+int wl_by_products(sun_lattice* lat, int rmax, int tmax, const Field& lines, double2* part, const int* state,
+                   double2* res, hipStream_t s) {
+    const Geom& g = lat->g;
+    const int nb[3] = {0, 0, monitor_blocks(g)};
+    for (int r = 0; r <= rmax; r++) {
+        HIP_TRY(lat->ops->wl_lines(lat->f, lines, g, r, state, s));
+        HIP_TRY(lat->ops->wl_loops(lat->f, lines, g, r, tmax, state, part, s));
+        HIP_TRY(launch_wl_finalize(part, nb, 1, tmax, wl_scale(lat), state, line_blocks(g),
+                                   res + (size_t)r * (tmax + 1), s));
+    }
+    return SUN_OK;
+}
+
+}  // namespace
+
 static int sun_wilson_loops_body(sun_lattice* lat, int rmax, int tmax, double* out, void* stream) {
     SUN_TRY(check_lattice(lat, "sun_wilson_loops"));
     if (!out) return fail(SUN_ERR_INVALID, "sun_wilson_loops: NULL output");
@@ -177,26 +237,37 @@ static int sun_wilson_loops_body(sun_lattice* lat, int rmax, int tmax, double* o
         return fail(SUN_ERR_INVALID, "sun_wilson_loops: rmax %d, tmax %d outside the lattice", rmax, tmax);
     hipStream_t s = pick_stream(lat, stream);
     HIP_TRY(hipSetDevice(lat->ctx->device));
-    const size_t full = (size_t)2 * lat->d.nc * lat->d.nc * (size_t)lat->d.precision;  // 18-real record
-    const size_t nline = 3 * (size_t)g.V;
-    const int nb = monitor_blocks(g);
-    const size_t npart = (size_t)3 * (tmax + 1) * nb;
-    const size_t nres = (size_t)(rmax + 1) * (tmax + 1);
-    DeviceScratch lines, part, res;
-    HIP_TRY(hipMalloc(&lines.p, nline * full));
-    HIP_TRY(hipMalloc(&part.p, npart * sizeof(double2)));
-    HIP_TRY(hipMalloc(&res.p, nres * sizeof(double2)));
-    const Field lf = make_field(lines.p, nline, full);
-    const double scale = 1.0 / (3.0 * lat->d.nc * (double)g.V);  // wilsonloop.cu:512
-    for (int r = 0; r <= rmax; r++) {
-        HIP_TRY(lat->ops->wl_lines(lat->f, lf, g, r, s));
-        HIP_TRY(lat->ops->wl_loops(lat->f, lf, g, r, tmax, (double2*)part.p, s));
-        HIP_TRY(launch_wl_finalize((const double2*)part.p, nb, tmax, scale, (double2*)res.p + (size_t)r * (tmax + 1),
-                                   s));
-    }
+    const size_t nres = (size_t)(rmax + 1) * (tmax + 1), res_bytes = (nres * sizeof(double2) + 255) & ~(size_t)255;
     std::vector<double2> h(nres);
-    HIP_TRY(hipMemcpyAsync(h.data(), res.p, nres * sizeof(double2), hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
+    const WlPlanes w = wl_planes(lat, tmax);
+    bool done = false;
+    if (w.fits()) {
+        constexpr size_t kPartBytes = size_t(64) << 20;  // of partial sums at a time
+        const size_t part = std::max(w.per_radius, std::min(w.per_radius * (rmax + 1), kPartBytes));
+        std::vector<int> st(line_blocks(g));
+        DeviceScratch mem;
+        HIP_TRY(hipMalloc(&mem.p, w.lines + part + res_bytes + st.size() * sizeof(int)));
+        char* p = static_cast<char*>(mem.p);
+        double2* res = (double2*)(p + w.lines);
+        int* state = (int*)(p + w.lines + res_bytes + part);
+        SUN_TRY(wl_by_planes(lat, w, rmax, tmax, (double*)p, (double2*)(p + w.lines + res_bytes), part, state, res, s));
+        HIP_TRY(hipMemcpyAsync(h.data(), res, nres * sizeof(double2), hipMemcpyDeviceToHost, s));
+        HIP_TRY(hipMemcpyAsync(st.data(), state, st.size() * sizeof(int), hipMemcpyDeviceToHost, s));
+        HIP_TRY(hipStreamSynchronize(s));
+        done = std::find(st.begin(), st.end(), kLinesBad) == st.end();
+    }
+    if (!done) {
+        const size_t full = (size_t)2 * lat->d.nc * lat->d.nc * (size_t)lat->d.precision;  // 18-real record
+        const size_t nline = 3 * (size_t)g.V;
+        DeviceScratch lines, part, res;
+        HIP_TRY(hipMalloc(&lines.p, nline * full));
+        HIP_TRY(hipMalloc(&part.p, (size_t)3 * (tmax + 1) * monitor_blocks(g) * sizeof(double2)));
+        HIP_TRY(hipMalloc(&res.p, res_bytes));
+        SUN_TRY(wl_by_products(lat, rmax, tmax, make_field(lines.p, nline, full), (double2*)part.p, nullptr,
+                               (double2*)res.p, s));
+        HIP_TRY(hipMemcpyAsync(h.data(), res.p, nres * sizeof(double2), hipMemcpyDeviceToHost, s));
+        HIP_TRY(hipStreamSynchronize(s));
+    }
     for (size_t i = 0; i < nres; i++) {
         out[2 * i] = h[i].x;
         out[2 * i + 1] = h[i].y;
@@ -208,11 +279,11 @@ extern "C" int sun_wilson_loops(sun_lattice* lat, int rmax, int tmax, double* ou
     return guard_alloc("sun_wilson_loops", [&] { return sun_wilson_loops_body(lat, rmax, tmax, out, stream); });
 }
 
-// The same kernels with the line field and the partial sums in the device's scratch
-// array (its address from sun_init) and the results written straight to the caller's
-// device buffer: no allocation and no host synchronisation.  The line field is set to
-// the identity by the r = 0 pass and every partial is written before it is read, so
-// nothing left in the array by an earlier call is used.
+// The same kernels with the lines and the partial sums in the device's scratch array (its
+// address from sun_init) and the results written straight to the caller's device buffer:
+// no allocation and no host synchronisation, so both routes are launched and the state of
+// the time lines decides on the device which one does anything.  Everything is written
+// before it is read, so nothing left in the array by an earlier call is used.
 extern "C" int sun_wilson_loops_noalloc(sun_lattice* lat, int rmax, int tmax, double* dev_out, void* stream) {
     SUN_TRY(check_lattice(lat, "sun_wilson_loops_noalloc"));
     if (!dev_out || (reinterpret_cast<uintptr_t>(dev_out) & 15u) != 0)
@@ -234,14 +305,15 @@ extern "C" int sun_wilson_loops_noalloc(sun_lattice* lat, int rmax, int tmax, do
     hipStream_t s = pick_stream(lat, stream);
     HIP_TRY(hipSetDevice(lat->ctx->device));
     unsigned char* base = static_cast<unsigned char*>(lat->ctx->scratch);
-    const Field lf = make_field(base, nline, full);
-    double2* part = reinterpret_cast<double2*>(base + line_bytes);
     double2* res = reinterpret_cast<double2*>(dev_out);
-    const double scale = 1.0 / (3.0 * lat->d.nc * (double)g.V);  // wilsonloop.cu:512
-    for (int r = 0; r <= rmax; r++) {
-        HIP_TRY(lat->ops->wl_lines(lat->f, lf, g, r, s));
-        HIP_TRY(lat->ops->wl_loops(lat->f, lf, g, r, tmax, part, s));
-        HIP_TRY(launch_wl_finalize(part, nb, tmax, scale, res + (size_t)r * (tmax + 1), s));
+    const WlPlanes w = wl_planes(lat, tmax);
+    int* state = nullptr;
+    if (w.fits() && w.lines + w.per_radius <= kNoAllocScratchBytes &&
+        line_blocks(g) * sizeof(int) <= kNoAllocStateBytes) {
+        state = reinterpret_cast<int*>(base + kNoAllocScratchBytes);
+        SUN_TRY(wl_by_planes(lat, w, rmax, tmax, reinterpret_cast<double*>(base),
+                             reinterpret_cast<double2*>(base + w.lines), kNoAllocScratchBytes - w.lines, state, res, s));
     }
-    return SUN_OK;
+    return wl_by_products(lat, rmax, tmax, make_field(base, nline, full), reinterpret_cast<double2*>(base + line_bytes),
+                          state, res, s);
 }

@@ -128,6 +128,37 @@ inline void batch_brick(const Geom& g, int& b1, int& b2, int& b3, int& spt) {
     spt = m;
 }
 
+// Wilson loops in (mu, t) planes: a workgroup of 256 threads takes `sites` spatial sites
+// with all times, two per thread, and T in chunks.  LDS: the moved lines of `extent` times
+// of each site (the lattice's and, going on around it, those that the last chunk reaches)
+// and the waves' sums.
+struct PlaneShape {
+    int sites, blocks, chunk, extent;
+    int sums, lds;  // bytes before the sums, and in all
+};
+// the shape for matrices of `bytes` bytes, or sites = 0 where the times do not fit
+inline PlaneShape plane_shape(const Geom& g, int T1, int bytes) {
+    constexpr int kThreads = 256, kLds = 156 * 1024;
+    PlaneShape p{};
+    // chunks of 5, 7 or 9 T (compiled kernels), as few as possible, then as small as possible
+    const int n = (T1 + 8) / 9, need = (T1 + n - 1) / n;
+    p.chunk = need <= 5 ? 5 : need <= 7 ? 7 : 9;
+    p.extent = g.X[3] + (n * p.chunk + 1) / 2 * 2;
+    const long long sums = 8ll * kThreads / 64 * 2 * T1;
+    const long long most = (kLds - sums) / ((long long)p.extent * bytes);
+    // two workgroups a CU where they fit
+    const long long two = (kLds / 2 - sums) / ((long long)p.extent * bytes);
+    long long sites = 2 * kThreads / g.X[3];
+    if (sites > most) sites = most;
+    if (two >= 1 && two < sites) sites = two;
+    if (sites < 1 || g.X[3] > 2 * kThreads) return p;
+    p.sites = (int)sites;
+    p.blocks = (g.str[3] + p.sites - 1) / p.sites;
+    p.sums = (p.extent * p.sites * bytes + 15) / 16 * 16;
+    p.lds = p.sums + (int)sums;
+    return p;
+}
+
 struct OpsTable {
     int nc, storage, real_bytes;
     // one (parity, mu) heatbath (hb=true) or overrelaxation launch
@@ -177,22 +208,30 @@ struct OpsTable {
     // box of temporal links, spatial copied (out 18-real)
     hipError_t (*multihit_ext)(const Field& in, const Field& out, const Geom&, uint64_t seed, int nhit, double bnc,
                                hipStream_t);
-    hipError_t (*wl_lines)(const Field& f, const Field& lines, const Geom&, int r, hipStream_t);
-    hipError_t (*wl_loops)(const Field& f, const Field& lines, const Geom&, int r, int tmax, double2* partials,
-                           hipStream_t);
+    // Wilson loops of radii [r_lo, r_hi) and T < T1, moved along time lines (planes, next =
+    // X3 + 1 times): 3 T1 blocks partials per radius, of the shape's blocks, ps[0] where the
+    // lines are unitary, ps[1] where not; nothing where they are kLinesBad
+    hipError_t (*wl_plane)(const Field& f, const Geom&, int r_lo, int r_hi, int T1, int next, const double* P,
+                           const int* state, const PlaneShape ps[2], double2* partials, hipStream_t);
+    // the same with the links multiplied out: the Wilson lines of radius r, then its loops;
+    // where state is given, only if it is kLinesBad
+    hipError_t (*wl_lines)(const Field& f, const Field& lines, const Geom&, int r, const int* state, hipStream_t);
+    hipError_t (*wl_loops)(const Field& f, const Field& lines, const Geom&, int r, int tmax, const int* state,
+                           double2* partials, hipStream_t);
     // operator-basis Wilson loops: the operator fields of direction mu at radius r
     // (family 0: 10 slots, 1: 25; slot k, V matrices of 2 N^2 reals one after another, at
     // ops + k * stride; rt8 = 2 sqrt 2)
     hipError_t (*wlop_fields)(const Field& f, char* ops, size_t stride, const Geom&, int family, int r,
                               int mu, double rt8, hipStream_t);
-    // time lines of every spatial site: P of `next` times, inverses Q (may be null) of X3
+    // time lines of every spatial site: P of `next` times (element by element where
+    // `planes`), inverses Q (may be null) of X3
     // times, FP64 N x N matrices; state[line_blocks(geom)]: per block whether its lines are
     // unitary (0), have condition numbers up to cond (1) or not (kLinesBad)
-    hipError_t (*time_lines)(const Field& f, const Geom&, int next, double cond, double* P, double* Q, int* state,
+    hipError_t (*time_lines)(const Field& f, const Geom&, int next, bool planes, double cond, double* P, double* Q, int* state,
                              hipStream_t);
     // the correlator of every slot pair; time lines of next = X3 + tmax times.  Partials:
     // [wlop_corr_blocks][T][i][j], or, where a state is kLinesBad,
-    // [(i nop + j)(tmax + 1) + T][monitor_blocks]
+    // [(i nop + j)(tmax + 1) + T][monitor_blocks]; state null: the latter, without lines
     hipError_t (*wlop_corr)(const Field& f, char* ops, size_t stride, const Geom&, int nop, int r, int mu,
                             int tmax, const double* P, const double* Q, const int* state, double* partials, hipStream_t);
     int max_block;   // largest workgroup the update kernels are compiled for
@@ -271,11 +310,14 @@ hipError_t launch_finalize(const double2* partials, int n, double scale0, double
 // scaled into out[0], out[1], recorded in history row ctr - first, then ctr += 1
 hipError_t launch_finalize_iteration(const double2* partials, int pb, int qb, double s_plaq, double s_poly,
                                      double2* out, double2* history, uint32_t* ctr, uint32_t first, hipStream_t s);
-// Wilson loops of one radius: out[T] = scale * sum over mu < 3 and the nb partials
-// of (mu, T), T = 0..tmax, in a fixed order
-hipError_t launch_wl_finalize(const double2* partials, int nb, int tmax, double scale, double2* out, hipStream_t s);
+// Wilson loops of nr radii: out[r (tmax + 1) + T] = scale * sum over mu < 3 and the partials
+// of (r, mu, T), T = 0..tmax, in a fixed order.  nb[i]: the workgroups of time lines in state
+// i; where nb[i] is 0 nothing is done.  state null: nb[kLinesBad].
+hipError_t launch_wl_finalize(const double2* partials, const int nb[3], int nr, int tmax, double scale,
+                              const int* state, int nstate, double2* out, hipStream_t s);
 // accum[(i nop + j) T1 + T] += the sum of the correlator's partials in a fixed order:
-// [rows][T][i][j], or [(i nop + j) T1 + T][nb] where one of the nstate states is kLinesBad
+// [rows][T][i][j], or [(i nop + j) T1 + T][nb] where one of the nstate states is kLinesBad or
+// state is null
 hipError_t launch_wlop_finalize(const double* partials, int rows, int nb, int nop, int T1, const int* state,
                                 int nstate, double* accum, hipStream_t s);
 // link monitor: out[0] = trace sum * scale_tr, out[1] = determinant sum * scale_det,

@@ -25,6 +25,7 @@ struct sun_wlop {
     void* ops = nullptr;    // nop slots
     double* partials = nullptr;
     int nb = 0, rows = 0;   // workgroups of the fallback and of the matrix-core correlator
+    bool direct = false;    // few T: without time lines
     double* lines = nullptr;   // time lines: X3 + tmax times of every spatial site
     double* inverses = nullptr;  // their inverses, X3 times
     int* state = nullptr;   // per block of lines, whether they are unitary or can be inverted
@@ -45,6 +46,15 @@ void release(sun_wlop* h) {
     if (h->state) hipFree(h->state);
     if (h->acc) hipFree(h->acc);
     delete h;
+}
+
+// Few T: multiplying every link out takes less time than moving the operators along time
+// lines (us per correlator, multiplied out / moved: FP64 A0, 16^3 x 32: 196 / 273 for two T,
+// 369 / 276 for four; 8^3 x 16: 44 / 61 and 53 / 61; FP32 A0, 16^4: 144 / 198 for six, 218 / 205
+// for nine; FP64 33 family, 16^3 x 32: 429 / 662 for one T, then more than moved).
+bool wlop_direct(int nop, int T1, int precision) {
+    if (nop > 16) return T1 <= 1;
+    return T1 <= (precision == SUN_PREC_F64 ? 3 : 8);
 }
 
 int check_radius(const sun_wlop* h, int r, int mu, const char* what) {
@@ -76,6 +86,7 @@ extern "C" int sun_wlop_create(sun_lattice* lat, int family, int tmax, sun_wlop*
     h->stride = (size_t)g.V * h->lb;
     h->nb = monitor_blocks(g);
     h->rows = wlop_corr_blocks(g);
+    h->direct = wlop_direct(nop, tmax + 1, lat->d.precision);
     const size_t nout = (size_t)nop * nop * (tmax + 1);
     HIP_TRY_CLEANUP(hipMalloc(&h->ops, (size_t)nop * h->stride), release(h));
     const size_t npart = nout * (size_t)std::max(h->nb, h->rows);
@@ -119,17 +130,18 @@ constexpr double kLineCond[2] = {4.0, 100.0};
 
 // the time lines of the lattice's present temporal links
 static int time_lines(sun_wlop* h, hipStream_t s) {
-    HIP_TRY(h->lat->ops->time_lines(h->lat->f, h->lat->g, h->lat->g.X[3] + h->tmax, kLineCond[h->lat->d.precision == SUN_PREC_F64], h->lines, h->inverses, h->state, s));
+    if (h->direct) return SUN_OK;
+    HIP_TRY(h->lat->ops->time_lines(h->lat->f, h->lat->g, h->lat->g.X[3] + h->tmax, false, kLineCond[h->lat->d.precision == SUN_PREC_F64], h->lines, h->inverses, h->state, s));
     return SUN_OK;
 }
 
 // the correlators of the current operator field, the time lines being there
 static int correlate(sun_wlop* h, int r, int mu, hipStream_t s) {
     sun_lattice* lat = h->lat;
-    HIP_TRY(lat->ops->wlop_corr(lat->f, (char*)h->ops, h->stride, lat->g, h->nop, r, mu, h->tmax, h->lines, h->inverses, h->state,
-                                h->partials, s));
-    HIP_TRY(launch_wlop_finalize(h->partials, h->rows, h->nb, h->nop, h->tmax + 1, h->state, line_blocks(lat->g), h->acc,
-                                 s));
+    HIP_TRY(lat->ops->wlop_corr(lat->f, (char*)h->ops, h->stride, lat->g, h->nop, r, mu, h->tmax, h->lines, h->inverses,
+                                h->direct ? nullptr : h->state, h->partials, s));
+    HIP_TRY(launch_wlop_finalize(h->partials, h->rows, h->nb, h->nop, h->tmax + 1,
+                                 h->direct ? nullptr : h->state, line_blocks(lat->g), h->acc, s));
     return SUN_OK;
 }
 

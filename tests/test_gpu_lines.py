@@ -59,3 +59,27 @@ def test_correlator_extents(ctx, oracle, dims, tmax, prec, family):
             got = ops.read()
     want = 2 * oracle.wlop_correlate(U, dims, oracle.wlop_fields(U, dims, family, r, mu), r, mu, tmax)
     assert np.abs(got - want).max() <= BAR[prec] * np.abs(want).max()
+
+
+@pytest.mark.parametrize("nc,prec", [(2, 8), (2, 4), (3, 8), (3, 4), (4, 8), (4, 4)])
+@pytest.mark.parametrize("kind", ["scattered", "singular"])
+def test_wilson_loops_of_non_unitary_lines(ctx, oracle, nc, prec, kind):
+    dims, rmax, tmax = (4, 2, 6, 8), 2, 8
+    with sun_amd.Lattice(ctx, nc, dims, BETAS[nc], 18, prec) as lat:
+        U = field(lat, oracle, nc, dims, kind)
+        got = lat.wilson_loops(rmax, tmax)
+    want = oracle.wilson_loops(U, dims, rmax, tmax)
+    assert np.abs(got - want).max() <= BAR[prec] * np.abs(want).max()
+
+
+@pytest.mark.parametrize("dims,tmax", [((2, 2, 2, 2), 2), ((2, 4, 2, 34), 34), ((4, 4, 4, 70), 17), ((6, 6, 4, 20), 0),
+                                       ((8, 6, 10, 6), 5), ((2, 2, 2, 516), 3)], ids=str)
+@pytest.mark.parametrize("storage,prec", [(18, 8), (12, 4)], ids=["f64", "f32"])
+def test_wilson_loops_extents(ctx, oracle, dims, tmax, storage, prec):
+    with sun_amd.Lattice(ctx, 3, dims, 6.0, storage, prec) as lat:
+        U = load_config(lat, thermalised(oracle, 3, dims, storage))
+        rmax = min(dims[:3])
+        got = lat.wilson_loops(rmax, tmax)
+        assert np.array_equal(got, lat.wilson_loops(rmax, tmax))
+    want = oracle.wilson_loops(U, dims, rmax, tmax)
+    assert np.abs(got - want).max() <= BAR[prec]
