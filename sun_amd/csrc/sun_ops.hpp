@@ -220,9 +220,11 @@ struct OpsTable {
                            double2* partials, hipStream_t);
     // operator-basis Wilson loops: the operator fields of direction mu at radius r
     // (family 0: 10 slots, 1: 25; slot k, V matrices of 2 N^2 reals one after another, at
-    // ops + k * stride; rt8 = 2 sqrt 2)
-    hipError_t (*wlop_fields)(const Field& f, char* ops, size_t stride, const Geom&, int family, int r,
-                              int mu, double rt8, hipStream_t);
+    // ops + k * stride; rt8 = 2 sqrt 2).  exact: FP64 fields with the reference's products one
+    // by one, otherwise from shared products (33: in kWlopAuxSlots more slots at aux; A0: slot
+    // 9 is left as it is)
+    hipError_t (*wlop_fields)(const Field& f, char* ops, char* aux, size_t stride, const Geom&, int family, int r,
+                              int mu, double rt8, bool exact, hipStream_t);
     // time lines of every spatial site: P of `next` times (element by element where
     // `planes`), inverses Q (may be null) of X3
     // times, FP64 N x N matrices; state[line_blocks(geom)]: per block whether its lines are
@@ -292,6 +294,8 @@ inline int partial_slots(const Geom& g) {
     const int a = 3 * monitor_blocks(g), b = plaquette_blocks(g) + polyakov_blocks(g);
     return a > b ? a : b;
 }
+// scratch slots of the 33 family's fields from shared products
+constexpr int kWlopAuxSlots = 14;
 // state of time lines that the measurement kernels cannot invert
 constexpr int kLinesBad = 2;
 // workgroups of the time-line kernel (64 spatial sites each)

@@ -23,6 +23,7 @@ struct sun_wlop {
     size_t lb = 0;          // bytes of one 18-real entry
     size_t stride = 0;      // bytes of one slot (V entries)
     void* ops = nullptr;    // nop slots
+    void* aux = nullptr;    // scratch slots of the 33 family
     double* partials = nullptr;
     int nb = 0, rows = 0;   // workgroups of the fallback and of the matrix-core correlator
     bool direct = false;    // few T: without time lines
@@ -40,6 +41,7 @@ int wlop_nops(int family) { return family == SUN_WLOP_A0 ? 10 : (family == SUN_W
 void release(sun_wlop* h) {
     if (!h) return;
     if (h->ops) hipFree(h->ops);
+    if (h->aux) hipFree(h->aux);
     if (h->partials) hipFree(h->partials);
     if (h->lines) hipFree(h->lines);
     if (h->inverses) hipFree(h->inverses);
@@ -89,6 +91,11 @@ extern "C" int sun_wlop_create(sun_lattice* lat, int family, int tmax, sun_wlop*
     h->direct = wlop_direct(nop, tmax + 1, lat->d.precision);
     const size_t nout = (size_t)nop * nop * (tmax + 1);
     HIP_TRY_CLEANUP(hipMalloc(&h->ops, (size_t)nop * h->stride), release(h));
+    if (family == SUN_WLOP_33) {
+        HIP_TRY_CLEANUP(hipMalloc(&h->aux, (size_t)kWlopAuxSlots * h->stride), release(h));
+    } else {  // slot 9 of A0 is zero throughout
+        HIP_TRY_CLEANUP(hipMemset((char*)h->ops + 9 * h->stride, 0, h->stride), release(h));
+    }
     const size_t npart = nout * (size_t)std::max(h->nb, h->rows);
     const size_t line = (size_t)2 * lat->d.nc * lat->d.nc * sizeof(double), vs = (size_t)g.str[3];
     HIP_TRY_CLEANUP(hipMalloc((void**)&h->partials, npart * sizeof(double)), release(h));
@@ -97,6 +104,7 @@ extern "C" int sun_wlop_create(sun_lattice* lat, int family, int tmax, sun_wlop*
     HIP_TRY_CLEANUP(hipMalloc((void**)&h->state, line_blocks(g) * sizeof(int)), release(h));
     HIP_TRY_CLEANUP(hipMalloc((void**)&h->acc, nout * sizeof(double)), release(h));
     HIP_TRY_CLEANUP(hipMemset(h->acc, 0, nout * sizeof(double)), release(h));
+    HIP_TRY_CLEANUP(hipStreamSynchronize(nullptr), release(h));  // the handle's streams do not wait for it
     *out = h;
     return SUN_OK;
 }
@@ -111,16 +119,22 @@ extern "C" int sun_wlop_destroy(sun_wlop* h) {
 
 extern "C" int sun_wlop_nops(const sun_wlop* h) { return h ? h->nop : 0; }
 
-extern "C" int sun_wlop_fields(sun_wlop* h, int r, int mu, void* stream) {
-    if (!h) return fail(SUN_ERR_INVALID, "sun_wlop_fields: NULL handle");
-    SUN_TRY(check_radius(h, r, mu, "sun_wlop_fields"));
+// exact: FP64 fields equal the products multiplied one by one, bit for bit
+static int fields(sun_wlop* h, int r, int mu, bool exact, hipStream_t s) {
     sun_lattice* lat = h->lat;
-    hipStream_t s = pick_stream(lat, stream);
-    HIP_TRY(hipSetDevice(lat->ctx->device));
-    HIP_TRY(lat->ops->wlop_fields(lat->f, (char*)h->ops, h->stride, lat->g, h->family, r, mu, 2.0 * std::sqrt(2.0), s));
+    HIP_TRY(lat->ops->wlop_fields(lat->f, (char*)h->ops, (char*)h->aux, h->stride, lat->g, h->family, r, mu,
+                                  2.0 * std::sqrt(2.0), exact, s));
     h->r = r;
     h->mu = mu;
     return SUN_OK;
+}
+
+extern "C" int sun_wlop_fields(sun_wlop* h, int r, int mu, void* stream) {
+    if (!h) return fail(SUN_ERR_INVALID, "sun_wlop_fields: NULL handle");
+    SUN_TRY(check_radius(h, r, mu, "sun_wlop_fields"));
+    hipStream_t s = pick_stream(h->lat, stream);
+    HIP_TRY(hipSetDevice(h->lat->ctx->device));
+    return fields(h, r, mu, true, s);
 }
 
 // Condition number up to which time lines are inverted, FP32 and FP64 lattices (whose X and
@@ -244,7 +258,7 @@ static int sun_wilson_loops_ops_body(sun_lattice* lat, int family, int rmax, int
     for (int r = 2; r <= rmax && rc == SUN_OK; r++) {
         rc = sun_wlop_clear(h, stream);
         for (int mu = 0; mu < 3 && rc == SUN_OK; mu++) {
-            rc = sun_wlop_fields(h, r, mu, stream);
+            rc = fields(h, r, mu, false, s);
             if (rc == SUN_OK) rc = correlate(h, r, mu, s);
         }
         if (rc == SUN_OK) rc = sun_wlop_read(h, out + (size_t)(r - 2) * n, stream);

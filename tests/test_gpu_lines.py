@@ -83,3 +83,16 @@ def test_wilson_loops_extents(ctx, oracle, dims, tmax, storage, prec):
         assert np.array_equal(got, lat.wilson_loops(rmax, tmax))
     want = oracle.wilson_loops(U, dims, rmax, tmax)
     assert np.abs(got - want).max() <= BAR[prec]
+
+
+@pytest.mark.parametrize("family,dims,rmax", [(0, (6, 6, 4, 10), 4), (1, (6, 6, 4, 10), 4), (0, (2, 2, 2, 6), 2),
+                                              (1, (2, 2, 2, 6), 2)], ids=str)
+@pytest.mark.parametrize("nc,storage,prec", [(2, 18, 8), (3, 18, 8), (3, 12, 4), (4, 18, 4)])
+def test_operator_loops_of_ragged_volumes(ctx, oracle, family, dims, rmax, nc, storage, prec):
+    """the fields from shared products: volumes that are no multiple of 64 or 256 sites, radii up
+    to the extent, sides of eight links around extents of 2, 4 and 6"""
+    with sun_amd.Lattice(ctx, nc, dims, BETAS[nc], storage, prec) as lat:
+        U = load_config(lat, thermalised(oracle, nc, dims, storage))
+        got = lat.wilson_loops_ops(rmax, 5, family)
+    want = oracle.wilson_loops_ops(U, dims, rmax, 5, family)
+    assert np.abs(got - want).max() <= (1e-12 if prec == 8 else 2e-5)
