@@ -162,6 +162,13 @@ Field sun::make_field(void* base, size_t nrec, size_t lb) {
     return f;
 }
 
+// the tuner's launch shapes, or the default ones
+static void set_launches(sun_lattice* L) {
+    Tuner& t = L->ctx->tuner;
+    L->cfg_hb = t.has("heatbath", L->d) ? t.lookup("heatbath", L->d) : default_launch(L->ops, L->g, 0);
+    L->cfg_or = t.has("overrelax", L->d) ? t.lookup("overrelax", L->d) : default_launch(L->ops, L->g, 1);
+}
+
 static void set_planes(sun_lattice* L) { L->f = make_field(L->buf, 4 * (size_t)L->g.V, link_bytes(&L->d)); }
 
 extern "C" size_t sun_lattice_bytes(const sun_lattice_desc* d) {
@@ -213,8 +220,7 @@ int sun::lattice_alloc(sun_ctx* ctx, const sun_lattice_desc* d, sun_lattice** ou
         lattice_free(L);
         return fail(SUN_ERR_HIP, "clearing link field: %s", hipGetErrorString(e));
     }
-    L->cfg_hb = ctx->tuner.lookup("heatbath", *d);
-    L->cfg_or = ctx->tuner.lookup("overrelax", *d);
+    set_launches(L);
     L->tuned = ctx->tuner.has("heatbath", *d) && ctx->tuner.has("overrelax", *d);
     *out = L;
     return SUN_OK;
@@ -256,8 +262,7 @@ int sun::lattice_in_memory(sun_ctx* ctx, const sun_lattice_desc* d, char* mem, i
     p += align256(sizeof(uint32_t));
     L->hist = (double2*)p;
     set_planes(L);
-    L->cfg_hb = ctx->tuner.lookup("heatbath", *d);
-    L->cfg_or = ctx->tuner.lookup("overrelax", *d);
+    set_launches(L);
     L->tuned = true;  // server lattices never tune: tuning needs a scratch copy outside the budget
     *out = L;
     return SUN_OK;
