@@ -307,7 +307,8 @@ typedef struct {
     int n_or;
     int reunit_every;
     int measure;     /* 0: no observables, 1: plaquette + Polyakov each iteration */
-    int use_graph;   /* capture one iteration in a hipGraph and replay it           */
+    int use_graph;   /* capture one iteration in a hipGraph and replay it (from 24
+                        iterations on; fewer are launched, capturing takes longer) */
 } sun_generate_desc;
 int sun_generate(sun_lattice *lat, const sun_generate_desc *desc, void *stream, double *obs);
 
@@ -330,7 +331,8 @@ int sun_batch_overrelax(sun_batch *b, void *stream);
 int sun_batch_reunitarize(sun_batch *b, void *stream);
 /* out: double[2*n] plaquette (spatial, temporal) per lattice, blocking */
 int sun_batch_plaquette(sun_batch *b, void *stream, double *out);
-/* n_iter x (HB + n_or OR [+ reunit]); hipGraph-captured when use_graph; per-lattice
+/* n_iter x (HB + n_or OR [+ reunit]); hipGraph-captured when use_graph (from 24
+ * iterations on); per-lattice
  * plaquette of every iteration into obs (host, n_iter*2*n doubles, may be NULL).
  * Chunks of lattices run on the caller's stream and two streams of the batch, which
  * wait for the caller's stream first and which it waits for at the end. */

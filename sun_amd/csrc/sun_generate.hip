@@ -17,6 +17,14 @@ using namespace sun;
 
 namespace {
 
+// Iterations from which a call that asks for a graph gets one.  Capturing and instantiating
+// the ~45 launches of an iteration takes ~0.55 ms, a replay saves at most ~0.7 us per launch
+// against launching them (8^4, 1 + 4 sweeps, us per call, graph / launches: 2 iterations 1139 /
+// 578, 8 2431 / 2091, 16 4277 / 4148; the lines cross at about 20.  32^4: 4136 / 3576, 14744 /
+// 14135, 28843 / 28238, no difference per iteration.  20 lattices 8^4 to 24^4: 8184 / 7543 for
+// two, 120939 / 118666 for 32).
+constexpr int kGraphIters = 24;
+
 struct GraphGuard {
     hipGraph_t g = nullptr;
     hipGraphExec_t x = nullptr;
@@ -92,7 +100,7 @@ static int sun_generate_body(sun_lattice* lat, const sun_generate_desc* d, void*
     HIP_TRY(hipMemcpyAsync(lat->sweep_dev, &first, sizeof(uint32_t), hipMemcpyHostToDevice, s));
     HIP_TRY(hipStreamSynchronize(s));
 
-    if (d->use_graph) {
+    if (d->use_graph && d->n_iter >= kGraphIters) {
         GraphGuard plain, with_reunit;
         const bool need_plain = d->reunit_every != 1;
         const bool need_reunit = d->reunit_every >= 1;
@@ -450,7 +458,7 @@ static int sun_batch_generate_body(sun_batch* b, uint32_t first_sweep, int n_ite
     const uint32_t zero = 0;
     HIP_TRY(hipMemcpyAsync(b->iter_dev, &zero, sizeof(uint32_t), hipMemcpyHostToDevice, s));
     HIP_TRY(hipStreamSynchronize(s));
-    if (use_graph) {
+    if (use_graph && n_iter >= kGraphIters) {
         GraphGuard plain, with_reunit;
         if (reunit_every != 1) SUN_TRY(capture(s, plain, [&] { return batch_iteration(b, n_or, false, measure, s); }));
         if (reunit_every >= 1)

@@ -1,0 +1,45 @@
+"""Long generation calls replay a captured iteration (shorter ones launch it): the same rows and
+links as without a graph, for one lattice (with both kinds of iterations) and for a batch over
+several streams, replayed in two calls with eager work between them."""
+import numpy as np
+import pytest
+
+import sun_amd
+
+pytestmark = pytest.mark.gpu
+
+ITERS = 30
+
+
+@pytest.mark.parametrize("nc,storage,prec", [(2, 18, 4), (3, 12, 4), (3, 18, 8)])
+def test_long_calls_replay_a_graph(ctx, nc, storage, prec):
+    beta = {2: 2.4, 3: 6.0}[nc]
+    out = []
+    for graph in (False, True):
+        with sun_amd.Lattice(ctx, nc, (4, 6, 4, 8), beta, storage, prec) as lat:
+            lat.cold_start()
+            every = 1 if storage == 12 else 3
+            rows = [lat.generate(7, ITERS, n_or=1, reunit_every=every, use_graph=graph)]
+            lat.heatbath(7, 1000)
+            rows.append(lat.generate(7, ITERS, n_or=1, reunit_every=every, first_sweep=ITERS, use_graph=graph))
+            out.append((rows, lat.to_host()))
+    assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
+
+
+def test_long_batch_calls_replay_a_graph(ctx):
+    dims = [(4, 4, 4, 4), (6, 4, 4, 8), (8, 8, 8, 8), (4, 4, 6, 6)]
+    out = []
+    for graph in (False, True):
+        lats = [sun_amd.Lattice(ctx, 3, d, 5.9, 12, 4) for d in dims]
+        for lat in lats:
+            lat.cold_start()
+        batch = sun_amd.Batch(ctx, lats, [3, 4, 5, 6])
+        rows = [batch.generate(0, ITERS, n_or=1, use_graph=graph)]
+        batch.overrelax()
+        rows.append(batch.generate(ITERS, ITERS, n_or=1, use_graph=graph))
+        out.append((rows, [lat.to_host() for lat in lats]))
+        batch.close()
+        for lat in lats:
+            lat.close()
+    assert np.array_equal(out[0][0], out[1][0])
+    assert all(np.array_equal(a, b) for a, b in zip(out[0][1], out[1][1]))
