@@ -221,8 +221,11 @@ SUN_HD void overrelax_link(Mat<R, N>& U, const Mat<R, N>& F) {
 // (projectlink.h:119-139), the reference's N = 3 choice, is this with w = 1,
 // tol = 0 and the blocks (0,1), (1,2), (0,2); it has no zero-block guard (a block
 // of exactly zero norm would give NaN there and the identity block here).
+// In FP32 with a tolerance the stop is decided by the rounding of the trace (1e-7 against
+// tolerances of 1e-10), so every rounding counts: project_link_rounded keeps the separately
+// rounded steps.
 template <typename R, int N>
-SUN_HD R retrace_conj(const Mat<R, N>& a, const Mat<R, N>& b) {  // Re Tr(a b) with b stored daggered
+SUN_HD R retrace_rounded(const Mat<R, N>& a, const Mat<R, N>& b) {  // Re Tr(a b) with b stored daggered
     R s = R(0);
 #pragma unroll
     for (int i = 0; i < N; i++)
@@ -232,10 +235,10 @@ SUN_HD R retrace_conj(const Mat<R, N>& a, const Mat<R, N>& b) {  // Re Tr(a b) w
 }
 
 template <typename R, int N>
-SUN_HD void project_link(Mat<R, N>& w, const Mat<R, N>& q_in, int nhit, R tol) {
+SUN_HD void project_link_rounded(Mat<R, N>& w, const Mat<R, N>& q_in, int nhit, R tol) {
     const Mat<R, N> q = dagger(q_in);
     R conver = R(1), old_tr = R(0);
-    if (tol > R(0)) old_tr = retrace_conj<R, N>(w, q) / R(N);
+    if (tol > R(0)) old_tr = retrace_rounded<R, N>(w, q) / R(N);
 #pragma unroll 1
     for (int hit = 0; hit < nhit && conver > tol; hit++) {
         // unrolled: compile-time rows keep w in registers
@@ -255,6 +258,101 @@ SUN_HD void project_link(Mat<R, N>& w, const Mat<R, N>& q_in, int nhit, R tol) {
             r.a[2] *= -k;
             r.a[3] *= -k;
             mul_block<R, N>(r, w, x, y);
+        }
+        if (tol > R(0)) {
+            const R new_tr = retrace_rounded<R, N>(w, q) / R(N);
+            conver = (new_tr - old_tr) / old_tr;
+            old_tr = new_tr;
+        }
+    }
+}
+
+// Otherwise fused multiply-adds throughout, and 1/|r| by the hardware's reciprocal square root
+// (FP64 with a correction step to full precision).  The hits are a serial chain of arithmetic
+// that bounds the smearing kernels: 3 x ~105 instructions per SU(3) hit, half of the separately
+// rounded form with its square root and division.
+template <typename R, int N>
+SUN_HD R retrace_conj(const Mat<R, N>& a, const Mat<R, N>& b) {  // Re Tr(a b) with b stored daggered
+    R s = R(0);
+#pragma unroll
+    for (int i = 0; i < N; i++)
+#pragma unroll
+        for (int j = 0; j < N; j++) s = fma(a.e[i][j].im, b.e[i][j].im, fma(a.e[i][j].re, b.e[i][j].re, s));
+    return s;
+}
+
+SUN_HD double inv_sqrt(double x) {
+#ifdef __HIP_DEVICE_COMPILE__
+    if (x > 1e-290 && x < 1e290) {
+        const double y = __builtin_amdgcn_rsq(x), e = fma(-x * y, y, 1.0);
+        return fma(y * e, fma(0.375, e, 0.5), y);
+    }
+#endif
+    return 1.0 / sqrt(x);
+}
+SUN_HD float inv_sqrt(float x) {
+    if (x < 1e-30f) return 1e15f * f32_rsq(x * 1e30f);  // the native instruction flushes denormals
+    return f32_rsq(x);
+}
+
+// 2 Re and Im combinations of the (x, y) block of w q (get_block_su2 of the product)
+template <typename R, int N>
+SUN_HD Quat<R> product_block(const Mat<R, N>& w, const Mat<R, N>& q, int x, int y) {
+    R r0 = R(0), r1 = R(0), r2 = R(0), r3 = R(0);
+#pragma unroll
+    for (int k = 0; k < N; k++) {
+        const cplx<R> a = w.e[x][k], b = w.e[y][k], c = q.e[k][x], d = q.e[k][y];
+        r0 = fma(-b.im, d.im, fma(b.re, d.re, fma(-a.im, c.im, fma(a.re, c.re, r0))));
+        r1 = fma(b.im, c.re, fma(b.re, c.im, fma(a.im, d.re, fma(a.re, d.im, r1))));
+        r2 = fma(b.im, c.im, fma(-b.re, c.re, fma(-a.im, d.im, fma(a.re, d.re, r2))));
+        r3 = fma(-b.im, d.re, fma(-b.re, d.im, fma(a.im, c.re, fma(a.re, c.im, r3))));
+    }
+    return Quat<R>{{r0, r1, r2, r3}};
+}
+
+// rows x, y of w <- u times them (mul_block)
+template <typename R, int N>
+SUN_HD void rotate_rows(const Quat<R>& u, Mat<R, N>& w, int x, int y) {
+    const R u0 = u.a[0], u1 = u.a[1], u2 = u.a[2], u3 = u.a[3];
+#pragma unroll
+    for (int j = 0; j < N; j++) {
+        const cplx<R> a = w.e[x][j], b = w.e[y][j];
+        w.e[x][j] = mk<R>(fma(-u1, b.im, fma(u2, b.re, fma(-u3, a.im, u0 * a.re))),
+                          fma(u1, b.re, fma(u2, b.im, fma(u3, a.re, u0 * a.im))));
+        w.e[y][j] = mk<R>(fma(u3, b.im, fma(u0, b.re, fma(-u1, a.im, -u2 * a.re))),
+                          fma(-u3, b.re, fma(u0, b.im, fma(u1, a.re, -u2 * a.im))));
+    }
+}
+
+template <typename R, int N>
+SUN_HD void project_link(Mat<R, N>& w, const Mat<R, N>& q_in, int nhit, R tol) {
+    if constexpr (sizeof(R) == 4) {
+        if (tol > R(0)) {
+            project_link_rounded<R, N>(w, q_in, nhit, tol);
+            return;
+        }
+    }
+    const Mat<R, N> q = dagger(q_in);
+    R conver = R(1), old_tr = R(0);
+    if (tol > R(0)) old_tr = retrace_conj<R, N>(w, q) / R(N);
+#pragma unroll 1
+    for (int hit = 0; hit < nhit && conver > tol; hit++) {
+        // unrolled: compile-time rows keep w in registers
+#pragma unroll
+        for (int block = 0; block < N * (N - 1) / 2; block++) {
+            const int x = block_p(N, block), y = block_q(N, block);
+            Quat<R> r = product_block<R, N>(w, q, x, y);
+            const R n2 = fma(r.a[3], r.a[3], fma(r.a[2], r.a[2], fma(r.a[1], r.a[1], r.a[0] * r.a[0])));
+            if (n2 == R(0)) {
+                r.a[0] = R(1);
+            } else {
+                const R k = inv_sqrt(n2);
+                r.a[0] *= k;
+                r.a[1] *= -k;
+                r.a[2] *= -k;
+                r.a[3] *= -k;
+            }
+            rotate_rows<R, N>(r, w, x, y);
         }
         if (tol > R(0)) {
             const R new_tr = retrace_conj<R, N>(w, q) / R(N);
