@@ -67,6 +67,90 @@ int lookup_scratch(int device, void** ptr) {
 }
 }  // namespace
 
+sun::Workspaces::Block sun::Workspaces::remove(int i) {
+    const Block b = idle_[i];
+    held_ -= b.bytes;
+    n_--;
+    for (; i < n_; i++) idle_[i] = idle_[i + 1];
+    return b;
+}
+
+hipError_t sun::Workspaces::take(size_t bytes, void** p, size_t* got) {
+    {
+        std::lock_guard<std::mutex> lk(mu_);
+        int best = -1;
+        for (int i = 0; i < n_; i++)
+            if (idle_[i].bytes >= bytes && idle_[i].bytes / 2 <= bytes &&
+                (best < 0 || idle_[i].bytes < idle_[best].bytes))
+                best = i;
+        if (best >= 0) {
+            const Block b = remove(best);
+            *p = b.p;
+            *got = b.bytes;
+            return hipSuccess;
+        }
+    }
+    *got = bytes;
+    return allocate(p, bytes);
+}
+
+void sun::Workspaces::give(void* p, size_t bytes) {
+    Block out[kBlocks + 1];
+    int n = 0;
+    if (bytes > kKeep) {
+        out[n++] = {p, bytes};
+    } else {
+        std::lock_guard<std::mutex> lk(mu_);
+        while (n_ == kBlocks || held_ + bytes > kKeep) out[n++] = remove(0);
+        idle_[n_++] = {p, bytes};
+        held_ += bytes;
+    }
+    for (int i = 0; i < n; i++) hipFree(out[i].p);
+}
+
+void sun::Workspaces::trim() {
+    Block out[kBlocks];
+    int n = 0;
+    {
+        std::lock_guard<std::mutex> lk(mu_);
+        while (n_) out[n++] = remove(n_ - 1);
+    }
+    for (int i = 0; i < n; i++) hipFree(out[i].p);
+}
+
+hipError_t sun::Workspaces::allocate(void** p, size_t bytes) {
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipErrorOutOfMemory) {
+        hipGetLastError();
+        trim();
+        e = hipMalloc(p, bytes);
+    }
+    return e;
+}
+
+hipError_t sun::CallScratch::take(size_t bytes) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s_, &st) != hipSuccess || st != hipStreamCaptureStatusNone) {
+        hipGetLastError();
+        return hipMalloc(&p_, bytes);
+    }
+    return ctx_->spare.take(bytes, &p_, &bytes_);
+}
+
+hipError_t sun::CallScratch::sync() {
+    const hipError_t e = hipStreamSynchronize(s_);
+    done_ = e == hipSuccess;
+    return e;
+}
+
+sun::CallScratch::~CallScratch() {
+    if (!p_) return;
+    if (bytes_ && (done_ || hipStreamSynchronize(s_) == hipSuccess))
+        ctx_->spare.give(p_, bytes_);
+    else
+        hipFree(p_);
+}
+
 extern "C" int sun_init(int device, int verbosity, int tune, sun_ctx** out) {
     if (!out) return fail(SUN_ERR_INVALID, "sun_init: out is NULL");
     *out = nullptr;
@@ -107,6 +191,7 @@ extern "C" int sun_finalize(sun_ctx* ctx) {
     hipSetDevice(ctx->device);
     hipStreamSynchronize(ctx->stream);
     ctx->tuner.save();
+    ctx->spare.trim();
     hipStreamDestroy(ctx->stream);
     delete ctx;
     return SUN_OK;
@@ -195,7 +280,7 @@ int sun::lattice_alloc(sun_ctx* ctx, const sun_lattice_desc* d, sun_lattice** ou
     const int tail = (int)(lb % 16);
     L->bytes = nl * lb;
     HIP_TRY_CLEANUP(hipSetDevice(ctx->device), delete L);
-    hipError_t e = hipMalloc(&L->buf, L->bytes);
+    hipError_t e = ctx->spare.allocate(&L->buf, L->bytes);
     if (e != hipSuccess) {
         delete L;
         hipGetLastError();
@@ -318,15 +403,13 @@ extern "C" int sun_lattice_convert(sun_lattice* dst, const sun_lattice* src, voi
     // (12/8-real reconstructed) and widened, then encoded in the destination's storage
     // and precision -- the same two kernels as a host round trip, without the host
     const size_t n = 4 * (size_t)src->g.V * src->d.nc * src->d.nc * 2;
-    double* tmp = nullptr;
-    HIP_TRY(hipMalloc(&tmp, n * sizeof(double)));
-    int rc = SUN_OK;
-    hipError_t e = src->ops->to_canonical(src->f, 4 * src->g.V, tmp, s);
-    if (e == hipSuccess) e = dst->ops->from_canonical(dst->f, 4 * dst->g.V, tmp, s);
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
-    if (e != hipSuccess) rc = fail(SUN_ERR_HIP, "sun_lattice_convert: %s", hipGetErrorString(e));
-    hipFree(tmp);
-    return rc;
+    CallScratch tmp(dst->ctx, s);
+    HIP_TRY(tmp.take(n * sizeof(double)));
+    hipError_t e = src->ops->to_canonical(src->f, 4 * src->g.V, (double*)tmp.at(), s);
+    if (e == hipSuccess) e = dst->ops->from_canonical(dst->f, 4 * dst->g.V, (double*)tmp.at(), s);
+    if (e == hipSuccess) e = tmp.sync();
+    if (e != hipSuccess) return fail(SUN_ERR_HIP, "sun_lattice_convert: %s", hipGetErrorString(e));
+    return SUN_OK;
 }
 
 extern "C" int sun_lattice_get_launch(const sun_lattice* lat, int kernel, sun_launch* out) {
@@ -573,32 +656,28 @@ extern "C" int sun_links_to_host(sun_lattice* lat, double* host, int layout) {
     if (!lat || !host) return fail(SUN_ERR_INVALID, "sun_links_to_host: NULL argument");
     if (layout != SUN_LAYOUT_CANONICAL) return fail(SUN_ERR_UNSUPPORTED, "layout %d", layout);
     const size_t n = 4 * (size_t)lat->g.V * lat->d.nc * lat->d.nc * 2;
-    double* tmp = nullptr;
     hipStream_t s = lat->ctx->stream;
-    HIP_TRY(hipMalloc(&tmp, n * sizeof(double)));
-    int rc = SUN_OK;
-    hipError_t e = lat->ops->to_canonical(lat->f, 4 * lat->g.V, tmp, s);
-    if (e == hipSuccess) e = hipMemcpyAsync(host, tmp, n * sizeof(double), hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
-    if (e != hipSuccess) rc = fail(SUN_ERR_HIP, "sun_links_to_host: %s", hipGetErrorString(e));
-    hipFree(tmp);
-    return rc;
+    CallScratch tmp(lat->ctx, s);
+    HIP_TRY(tmp.take(n * sizeof(double)));
+    hipError_t e = lat->ops->to_canonical(lat->f, 4 * lat->g.V, (double*)tmp.at(), s);
+    if (e == hipSuccess) e = hipMemcpyAsync(host, tmp.at(), n * sizeof(double), hipMemcpyDeviceToHost, s);
+    if (e == hipSuccess) e = tmp.sync();
+    if (e != hipSuccess) return fail(SUN_ERR_HIP, "sun_links_to_host: %s", hipGetErrorString(e));
+    return SUN_OK;
 }
 
 extern "C" int sun_links_from_host(sun_lattice* lat, const double* host, int layout) {
     if (!lat || !host) return fail(SUN_ERR_INVALID, "sun_links_from_host: NULL argument");
     if (layout != SUN_LAYOUT_CANONICAL) return fail(SUN_ERR_UNSUPPORTED, "layout %d", layout);
     const size_t n = 4 * (size_t)lat->g.V * lat->d.nc * lat->d.nc * 2;
-    double* tmp = nullptr;
     hipStream_t s = lat->ctx->stream;
-    HIP_TRY(hipMalloc(&tmp, n * sizeof(double)));
-    int rc = SUN_OK;
-    hipError_t e = hipMemcpyAsync(tmp, host, n * sizeof(double), hipMemcpyHostToDevice, s);
-    if (e == hipSuccess) e = lat->ops->from_canonical(lat->f, 4 * lat->g.V, tmp, s);
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
-    if (e != hipSuccess) rc = fail(SUN_ERR_HIP, "sun_links_from_host: %s", hipGetErrorString(e));
-    hipFree(tmp);
-    return rc;
+    CallScratch tmp(lat->ctx, s);
+    HIP_TRY(tmp.take(n * sizeof(double)));
+    hipError_t e = hipMemcpyAsync(tmp.at(), host, n * sizeof(double), hipMemcpyHostToDevice, s);
+    if (e == hipSuccess) e = lat->ops->from_canonical(lat->f, 4 * lat->g.V, (double*)tmp.at(), s);
+    if (e == hipSuccess) e = tmp.sync();
+    if (e != hipSuccess) return fail(SUN_ERR_HIP, "sun_links_from_host: %s", hipGetErrorString(e));
+    return SUN_OK;
 }
 
 // ---------------------------------------------------------------------------------

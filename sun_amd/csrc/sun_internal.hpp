@@ -82,6 +82,38 @@ class Tuner {
 
 }  // namespace sun
 
+namespace sun {
+// Device memory for the length of a call (or of an operator handle): blocks that were given back
+// wait here for the next call.  hipMalloc and hipFree of a measurement's scratch cost 0.1 to 1.5 ms
+// a call, and a wait for memory freed just before; HYP smearing and Wilson loops of 16^3 x 32 SU(3)
+// FP64 (0.5 GB) took 3.8 to 15 ms with them and take 2.2 without.  At most kKeep bytes stay idle (a call that needs
+// more works for longer than the allocation takes), and all of them go back when an allocation of
+// the context fails and at sun_finalize.  A block is given back when the work on it is done, so
+// the next taker may use it on any stream.
+class Workspaces {
+public:
+    static constexpr size_t kKeep = size_t(2) << 30;
+    // an idle block of bytes to twice that, or a new one (its size in *got)
+    hipError_t take(size_t bytes, void** p, size_t* got);
+    void give(void* p, size_t bytes);
+    void trim();
+    // hipMalloc, once more without the idle blocks if it fails
+    hipError_t allocate(void** p, size_t bytes);
+
+private:
+    struct Block {
+        void* p;
+        size_t bytes;
+    };
+    static constexpr int kBlocks = 16;
+    std::mutex mu_;
+    Block idle_[kBlocks];  // oldest first
+    int n_ = 0;
+    size_t held_ = 0;
+    Block remove(int i);
+};
+}  // namespace sun
+
 struct sun_ctx {
     int device = 0;
     int verbosity = 0;
@@ -94,6 +126,7 @@ struct sun_ctx {
     // this device's copy of the allocation-free entry points' scratch array (its
     // device address, looked up once per device at sun_init)
     void* scratch = nullptr;
+    sun::Workspaces spare;
 };
 
 namespace sun {
@@ -106,6 +139,25 @@ constexpr size_t kNoAllocStateBytes = size_t(16) << 10;
 // device result slots of a lattice: plaquette and Polyakov of sun_generate, or the
 // three of the link monitor
 constexpr int kResSlots = 3;
+
+// A call's scratch on its stream.  sync() before the call returns; on an error path the
+// destructor waits.  A call under stream capture allocates, as it would without idle blocks.
+class CallScratch {
+public:
+    CallScratch(sun_ctx* ctx, hipStream_t s) : ctx_(ctx), s_(s) {}
+    CallScratch(const CallScratch&) = delete;
+    ~CallScratch();
+    hipError_t take(size_t bytes);
+    hipError_t sync();
+    char* at(size_t offset = 0) const { return static_cast<char*>(p_) + offset; }
+
+private:
+    sun_ctx* ctx_;
+    hipStream_t s_;
+    void* p_ = nullptr;
+    size_t bytes_ = 0;  // 0: not from the idle blocks
+    bool done_ = false;
+};
 }  // namespace sun
 
 struct sun_lattice {

@@ -3,9 +3,8 @@
 // HYP smearing (smear/hyp.cu:277-368), spatial multihit (smear/multihitsp.cu:246-266),
 // multihit of temporal links (smear/multihit.cu:291-333), extended multihit
 // (smear/multihitext.cu:395-459) and Wilson loops (meas/wilsonloop.cu:494-516).
-// Scratch (the ping-pong field of APE, the Wilson lines and partial sums) is
-// allocated per call: these are measurements between generation steps, not part
-// of the generation loop.
+// Scratch (the ping-pong field of APE, the Wilson lines and partial sums) is the
+// context's, taken for the length of a call.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -16,13 +15,6 @@
 using namespace sun;
 
 namespace {
-
-struct DeviceScratch {
-    void* p = nullptr;
-    ~DeviceScratch() {
-        if (p) hipFree(p);
-    }
-};
 
 int check_lattice(const sun_lattice* lat, const char* what) {
     if (!lat) return fail(SUN_ERR_INVALID, "%s: NULL lattice", what);
@@ -41,21 +33,21 @@ extern "C" int sun_ape_smear(sun_lattice* lat, double w, int steps, int nhit, do
     if (steps == 0) return SUN_OK;
     hipStream_t s = pick_stream(lat, stream);
     HIP_TRY(hipSetDevice(lat->ctx->device));
-    DeviceScratch tmp;
-    HIP_TRY(hipMalloc(&tmp.p, lat->bytes));
+    CallScratch tmp(lat->ctx, s);
+    HIP_TRY(tmp.take(lat->bytes));
     // ping-pong between the lattice and a copy: every direction of a step reads the
     // field of the previous step (ape.cu:209-214); the directions a step does not
     // smear are equal in both buffers
-    HIP_TRY(hipMemcpyAsync(tmp.p, lat->buf, lat->bytes, hipMemcpyDeviceToDevice, s));
-    const Field other = make_field(tmp.p, 4 * (size_t)lat->g.V, link_bytes(&lat->d));
+    HIP_TRY(hipMemcpyAsync(tmp.at(), lat->buf, lat->bytes, hipMemcpyDeviceToDevice, s));
+    const Field other = make_field(tmp.at(), 4 * (size_t)lat->g.V, link_bytes(&lat->d));
     for (int st = 0; st < steps; st++) {
         const Field& src = (st & 1) ? other : lat->f;
         const Field& dst = (st & 1) ? lat->f : other;
         for (int mu = time_dir ? 3 : 0; mu < (time_dir ? 4 : 3); mu++)
             HIP_TRY(lat->ops->ape(src, dst, lat->g, mu, w, nhit, tol, s));
     }
-    if (steps & 1) HIP_TRY(hipMemcpyAsync(lat->buf, tmp.p, lat->bytes, hipMemcpyDeviceToDevice, s));
-    HIP_TRY(hipStreamSynchronize(s));
+    if (steps & 1) HIP_TRY(hipMemcpyAsync(lat->buf, tmp.at(), lat->bytes, hipMemcpyDeviceToDevice, s));
+    HIP_TRY(tmp.sync());
     return SUN_OK;
 }
 
@@ -67,20 +59,20 @@ extern "C" int sun_stout_smear(sun_lattice* lat, double rho, int steps, int time
     if (steps == 0) return SUN_OK;
     hipStream_t s = pick_stream(lat, stream);
     HIP_TRY(hipSetDevice(lat->ctx->device));
-    DeviceScratch tmp;
-    HIP_TRY(hipMalloc(&tmp.p, lat->bytes));
+    CallScratch tmp(lat->ctx, s);
+    HIP_TRY(tmp.take(lat->bytes));
     // the ping-pong of sun_ape_smear: every direction of a step reads the previous
     // step's field (stout.cu:697-705)
-    HIP_TRY(hipMemcpyAsync(tmp.p, lat->buf, lat->bytes, hipMemcpyDeviceToDevice, s));
-    const Field other = make_field(tmp.p, 4 * (size_t)lat->g.V, link_bytes(&lat->d));
+    HIP_TRY(hipMemcpyAsync(tmp.at(), lat->buf, lat->bytes, hipMemcpyDeviceToDevice, s));
+    const Field other = make_field(tmp.at(), 4 * (size_t)lat->g.V, link_bytes(&lat->d));
     for (int st = 0; st < steps; st++) {
         const Field& src = (st & 1) ? other : lat->f;
         const Field& dst = (st & 1) ? lat->f : other;
         for (int mu = time_dir ? 3 : 0; mu < (time_dir ? 4 : 3); mu++)
             HIP_TRY(lat->ops->stout(src, dst, lat->g, mu, rho, s));
     }
-    if (steps & 1) HIP_TRY(hipMemcpyAsync(lat->buf, tmp.p, lat->bytes, hipMemcpyDeviceToDevice, s));
-    HIP_TRY(hipStreamSynchronize(s));
+    if (steps & 1) HIP_TRY(hipMemcpyAsync(lat->buf, tmp.at(), lat->bytes, hipMemcpyDeviceToDevice, s));
+    HIP_TRY(tmp.sync());
     return SUN_OK;
 }
 
@@ -96,31 +88,26 @@ extern "C" int sun_hyp_smear(sun_lattice* lat, double alpha1, double alpha2, dou
     HIP_TRY(hipSetDevice(lat->ctx->device));
     const size_t full = (size_t)2 * lat->d.nc * lat->d.nc * (size_t)lat->d.precision;  // 18-real record
     const size_t one = (size_t)lat->g.V * full;  // one pair's field
-    DeviceScratch tmp, bar, til, tab;
-    HIP_TRY(hipMalloc(&tmp.p, lat->bytes));
-    HIP_TRY(hipMalloc(&bar.p, 12 * one));
-    HIP_TRY(hipMalloc(&til.p, 12 * one));
-    // 12 separate V-link fields per level (site-indexed plane views), as a device table
     Field views[24];
-    for (int p = 0; p < 12; p++) {
-        views[p] = make_field((char*)bar.p + p * one, (size_t)lat->g.V, full);
-        views[12 + p] = make_field((char*)til.p + p * one, (size_t)lat->g.V, full);
-    }
-    HIP_TRY(hipMalloc(&tab.p, sizeof(views)));
-    HIP_TRY(hipMemcpy(tab.p, views, sizeof(views), hipMemcpyHostToDevice));
-    const Field* fb = (const Field*)tab.p;
+    const size_t at_tab = (lat->bytes + 255) & ~(size_t)255, at_pairs = at_tab + ((sizeof(views) + 255) & ~(size_t)255);
+    CallScratch tmp(lat->ctx, s);
+    HIP_TRY(tmp.take(at_pairs + 24 * one));
+    // 12 separate V-link fields per level (site-indexed plane views), as a device table
+    for (int p = 0; p < 24; p++) views[p] = make_field(tmp.at(at_pairs + p * one), (size_t)lat->g.V, full);
+    HIP_TRY(hipMemcpyAsync(tmp.at(at_tab), views, sizeof(views), hipMemcpyHostToDevice, s));
+    const Field* fb = (const Field*)tmp.at(at_tab);
     const Field* ft = fb + 12;
     // the ping-pong of sun_ape_smear (hyp.cu:291-313): each step reads the previous field
-    HIP_TRY(hipMemcpyAsync(tmp.p, lat->buf, lat->bytes, hipMemcpyDeviceToDevice, s));
-    const Field other = make_field(tmp.p, 4 * (size_t)lat->g.V, link_bytes(&lat->d));
+    HIP_TRY(hipMemcpyAsync(tmp.at(), lat->buf, lat->bytes, hipMemcpyDeviceToDevice, s));
+    const Field other = make_field(tmp.at(), 4 * (size_t)lat->g.V, link_bytes(&lat->d));
     for (int st = 0; st < steps; st++) {
         const Field& src = (st & 1) ? other : lat->f;
         const Field& dst = (st & 1) ? lat->f : other;
         HIP_TRY(lat->ops->hyp(src, fb, ft, dst, lat->g, time_dir ? 3 : 0, time_dir ? 4 : 3, alpha1, alpha2, alpha3,
                               nhit, tol, s));
     }
-    if (steps & 1) HIP_TRY(hipMemcpyAsync(lat->buf, tmp.p, lat->bytes, hipMemcpyDeviceToDevice, s));
-    HIP_TRY(hipStreamSynchronize(s));
+    if (steps & 1) HIP_TRY(hipMemcpyAsync(lat->buf, tmp.at(), lat->bytes, hipMemcpyDeviceToDevice, s));
+    HIP_TRY(tmp.sync());
     return SUN_OK;
 }
 
@@ -245,28 +232,28 @@ static int sun_wilson_loops_body(sun_lattice* lat, int rmax, int tmax, double* o
         constexpr size_t kPartBytes = size_t(64) << 20;  // of partial sums at a time
         const size_t part = std::max(w.per_radius, std::min(w.per_radius * (rmax + 1), kPartBytes));
         std::vector<int> st(line_blocks(g));
-        DeviceScratch mem;
-        HIP_TRY(hipMalloc(&mem.p, w.lines + part + res_bytes + st.size() * sizeof(int)));
-        char* p = static_cast<char*>(mem.p);
+        CallScratch mem(lat->ctx, s);
+        HIP_TRY(mem.take(w.lines + part + res_bytes + st.size() * sizeof(int)));
+        char* p = mem.at();
         double2* res = (double2*)(p + w.lines);
         int* state = (int*)(p + w.lines + res_bytes + part);
         SUN_TRY(wl_by_planes(lat, w, rmax, tmax, (double*)p, (double2*)(p + w.lines + res_bytes), part, state, res, s));
         HIP_TRY(hipMemcpyAsync(h.data(), res, nres * sizeof(double2), hipMemcpyDeviceToHost, s));
         HIP_TRY(hipMemcpyAsync(st.data(), state, st.size() * sizeof(int), hipMemcpyDeviceToHost, s));
-        HIP_TRY(hipStreamSynchronize(s));
+        HIP_TRY(mem.sync());
         done = std::find(st.begin(), st.end(), kLinesBad) == st.end();
     }
     if (!done) {
         const size_t full = (size_t)2 * lat->d.nc * lat->d.nc * (size_t)lat->d.precision;  // 18-real record
         const size_t nline = 3 * (size_t)g.V;
-        DeviceScratch lines, part, res;
-        HIP_TRY(hipMalloc(&lines.p, nline * full));
-        HIP_TRY(hipMalloc(&part.p, (size_t)3 * (tmax + 1) * monitor_blocks(g) * sizeof(double2)));
-        HIP_TRY(hipMalloc(&res.p, res_bytes));
-        SUN_TRY(wl_by_products(lat, rmax, tmax, make_field(lines.p, nline, full), (double2*)part.p, nullptr,
-                               (double2*)res.p, s));
-        HIP_TRY(hipMemcpyAsync(h.data(), res.p, nres * sizeof(double2), hipMemcpyDeviceToHost, s));
-        HIP_TRY(hipStreamSynchronize(s));
+        const size_t at_part = (nline * full + 255) & ~(size_t)255;
+        const size_t at_res = at_part + (size_t)3 * (tmax + 1) * monitor_blocks(g) * sizeof(double2);
+        CallScratch mem(lat->ctx, s);
+        HIP_TRY(mem.take(at_res + res_bytes));
+        SUN_TRY(wl_by_products(lat, rmax, tmax, make_field(mem.at(), nline, full), (double2*)mem.at(at_part), nullptr,
+                               (double2*)mem.at(at_res), s));
+        HIP_TRY(hipMemcpyAsync(h.data(), mem.at(at_res), nres * sizeof(double2), hipMemcpyDeviceToHost, s));
+        HIP_TRY(mem.sync());
     }
     for (size_t i = 0; i < nres; i++) {
         out[2 * i] = h[i].x;

@@ -712,7 +712,7 @@ extern "C" int sun_server_create(sun_ctx* ctx, size_t budget, int max_jobs, sun_
     S->budget = budget;
     S->max_jobs = max_jobs;
     HIP_TRY_CLEANUP(hipSetDevice(ctx->device), delete S);
-    const hipError_t e = hipMalloc(&S->base, budget);
+    const hipError_t e = ctx->spare.allocate((void**)&S->base, budget);
     if (e != hipSuccess) {
         hipGetLastError();
         delete S;

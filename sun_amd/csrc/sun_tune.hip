@@ -123,7 +123,7 @@ int tune_lattice(sun_lattice* lat, hipStream_t s) {
     sun_ctx* ctx = lat->ctx;
     if (!ctx->tuner.enabled() || lat->tuned) return SUN_OK;
     void* backup = nullptr;
-    HIP_TRY(hipMalloc(&backup, lat->bytes));
+    HIP_TRY(ctx->spare.allocate(&backup, lat->bytes));
     hipEvent_t e0 = nullptr, e1 = nullptr;
     int rc = SUN_OK;
     hipError_t e = hipMemcpyAsync(backup, lat->buf, lat->bytes, hipMemcpyDeviceToDevice, s);

@@ -22,6 +22,7 @@ struct sun_wlop {
     int family = 0, nop = 0, tmax = 0;
     size_t lb = 0;          // bytes of one 18-real entry
     size_t stride = 0;      // bytes of one slot (V entries)
+    size_t held = 0;        // bytes of the block that all the following lie in
     void* ops = nullptr;    // nop slots
     void* aux = nullptr;    // scratch slots of the 33 family
     double* partials = nullptr;
@@ -40,13 +41,12 @@ int wlop_nops(int family) { return family == SUN_WLOP_A0 ? 10 : (family == SUN_W
 
 void release(sun_wlop* h) {
     if (!h) return;
-    if (h->ops) hipFree(h->ops);
-    if (h->aux) hipFree(h->aux);
-    if (h->partials) hipFree(h->partials);
-    if (h->lines) hipFree(h->lines);
-    if (h->inverses) hipFree(h->inverses);
-    if (h->state) hipFree(h->state);
-    if (h->acc) hipFree(h->acc);
+    if (h->ops) {
+        if (hipDeviceSynchronize() == hipSuccess)
+            h->lat->ctx->spare.give(h->ops, h->held);
+        else
+            hipFree(h->ops);
+    }
     delete h;
 }
 
@@ -90,19 +90,30 @@ extern "C" int sun_wlop_create(sun_lattice* lat, int family, int tmax, sun_wlop*
     h->rows = wlop_corr_blocks(g);
     h->direct = wlop_direct(nop, tmax + 1, lat->d.precision);
     const size_t nout = (size_t)nop * nop * (tmax + 1);
-    HIP_TRY_CLEANUP(hipMalloc(&h->ops, (size_t)nop * h->stride), release(h));
-    if (family == SUN_WLOP_33) {
-        HIP_TRY_CLEANUP(hipMalloc(&h->aux, (size_t)kWlopAuxSlots * h->stride), release(h));
-    } else {  // slot 9 of A0 is zero throughout
-        HIP_TRY_CLEANUP(hipMemset((char*)h->ops + 9 * h->stride, 0, h->stride), release(h));
-    }
     const size_t npart = nout * (size_t)std::max(h->nb, h->rows);
     const size_t line = (size_t)2 * lat->d.nc * lat->d.nc * sizeof(double), vs = (size_t)g.str[3];
-    HIP_TRY_CLEANUP(hipMalloc((void**)&h->partials, npart * sizeof(double)), release(h));
-    HIP_TRY_CLEANUP(hipMalloc((void**)&h->lines, vs * (g.X[3] + tmax) * line), release(h));
-    HIP_TRY_CLEANUP(hipMalloc((void**)&h->inverses, vs * g.X[3] * line), release(h));
-    HIP_TRY_CLEANUP(hipMalloc((void**)&h->state, line_blocks(g) * sizeof(int)), release(h));
-    HIP_TRY_CLEANUP(hipMalloc((void**)&h->acc, nout * sizeof(double)), release(h));
+    size_t total = 0;
+    auto part = [&](size_t bytes) {
+        const size_t at = total;
+        total += (bytes + 255) & ~(size_t)255;
+        return at;
+    };
+    part((size_t)nop * h->stride);
+    const size_t at_aux = part(family == SUN_WLOP_33 ? (size_t)kWlopAuxSlots * h->stride : 0);
+    const size_t at_partials = part(npart * sizeof(double)), at_lines = part(vs * (g.X[3] + tmax) * line);
+    const size_t at_inverses = part(vs * g.X[3] * line), at_state = part(line_blocks(g) * sizeof(int));
+    const size_t at_acc = part(nout * sizeof(double));
+    HIP_TRY_CLEANUP(lat->ctx->spare.take(total, &h->ops, &h->held), release(h));
+    char* base = static_cast<char*>(h->ops);
+    if (family == SUN_WLOP_33)
+        h->aux = base + at_aux;
+    else  // slot 9 of A0 is zero throughout
+        HIP_TRY_CLEANUP(hipMemset(base + 9 * h->stride, 0, h->stride), release(h));
+    h->partials = (double*)(base + at_partials);
+    h->lines = (double*)(base + at_lines);
+    h->inverses = (double*)(base + at_inverses);
+    h->state = (int*)(base + at_state);
+    h->acc = (double*)(base + at_acc);
     HIP_TRY_CLEANUP(hipMemset(h->acc, 0, nout * sizeof(double)), release(h));
     HIP_TRY_CLEANUP(hipStreamSynchronize(nullptr), release(h));  // the handle's streams do not wait for it
     *out = h;
@@ -112,7 +123,6 @@ extern "C" int sun_wlop_create(sun_lattice* lat, int family, int tmax, sun_wlop*
 extern "C" int sun_wlop_destroy(sun_wlop* h) {
     if (!h) return SUN_OK;
     hipSetDevice(h->lat->ctx->device);
-    hipDeviceSynchronize();
     release(h);
     return SUN_OK;
 }
