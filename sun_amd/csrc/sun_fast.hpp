@@ -211,6 +211,29 @@ SUN_HD F3 staple_su3_rt(const Field& f, const Geom& g, int id, int parity, int m
     return S;
 }
 
+// one term of the staple sum: the upper or the lower path of the plane (mu, nu)
+template <int STORE>
+SUN_HD F3 staple_term_su3(const Field& f, uint32_t V, int mu, int nu, bool down, uint32_t self, uint32_t eo_pmu,
+                          uint32_t eo_nu, uint32_t eo_nu_pmu) {
+    const F3 B = load_rows<STORE>(f, (uint32_t)mu * V + eo_nu);
+    F3 A = load_rows<STORE>(f, (uint32_t)nu * V + (down ? eo_nu : self));
+    F3 Cc = load_rows<STORE>(f, (uint32_t)nu * V + (down ? eo_nu_pmu : eo_pmu));
+    need_row2<STORE>(Cc);
+    F3 W, T;
+    if (down) {
+        need_row2<STORE>(A);
+        mul_2r(B, Cc, W);
+        complete_row2(W);
+        mul_2r_adag(A, W, T);
+    } else {
+        mul_2r_bdag(B, Cc, W);
+        complete_row2(W);
+        mul_2r(A, W, T);
+    }
+    complete_row2(T);
+    return T;
+}
+
 // staple sum (monte.cu:63-80) for a compile-time direction MU.  With PREFETCH the
 // six links U_MU(x +- nu) are loaded first: each of them is needed by six sites
 // (y -+ nu), and issuing all six loads at the start of every thread puts those six
@@ -517,9 +540,7 @@ SUN_HD void overrelax_su3(F3& U, const F3& S) {
     }
 }
 
-SUN_HD void heatbath_su3(F3& U, const F3& S, double bnc, const DrawKey& key) {
-    // the counters of every block's first attempt and final draws are known now
-    const BlockDraws bd[3] = {BlockDraws(key, 0), BlockDraws(key, 1), BlockDraws(key, 2)};
+SUN_HD void heatbath_su3(F3& U, const F3& S, double bnc, const DrawKey& key, const BlockDraws bd[3]) {
 #pragma unroll
     for (int block = 0; block < 3; block++) {
         const int p = block_p(3, block), q = block_q(3, block);
@@ -534,6 +555,12 @@ SUN_HD void heatbath_su3(F3& U, const F3& S, double bnc, const DrawKey& key) {
         generate_su2_milc_f32(ap, key, block, bd[block], a.a);
         rotate_rows(U, mul_uv_dagger(a, r), p, q);
     }
+}
+
+SUN_HD void heatbath_su3(F3& U, const F3& S, double bnc, const DrawKey& key) {
+    // the counters of every block's first attempt and final draws are known now
+    const BlockDraws bd[3] = {BlockDraws(key, 0), BlockDraws(key, 1), BlockDraws(key, 2)};
+    heatbath_su3(U, S, bnc, key, bd);
 }
 
 // Re Tr(X Y^+) = sum_ij Re(X_ij conj(Y_ij))

@@ -115,6 +115,7 @@ struct DrawKey {
 struct BlockDraws {
     uint32_t first[4];
     uint32_t fin[2];
+    BlockDraws() = default;
     SUN_HD BlockDraws(const DrawKey& key, int block) {
         key.words((uint32_t)block * kBlockCounters, first);
         uint32_t t[4];
@@ -175,41 +176,68 @@ SUN_HD float f32_rcp(float x) {
 #endif
 }
 
+// What the double sampler below takes from the draws alone, whatever al is: of a
+// Kennedy-Pendleton attempt its numerator and comparison value, of the final draws
+// 2 u - 1 and the azimuth's sine and cosine.
+struct Attempt {
+    double num, x4;
+    Attempt() = default;
+    SUN_HD explicit Attempt(const uint32_t w[4]) {
+        double xr1 = u01(w[0]);
+        xr1 = sun_log(xr1 + 1.e-10);
+        double xr2 = u01(w[1]);
+        xr2 = sun_log(xr2 + 1.e-10);
+        double xr3 = u01(w[2]);
+        x4 = u01(w[3]);
+        xr3 = sun_cos2pi(xr3);
+        num = xr2 + xr1 * xr3 * xr3;
+    }
+    // d of the attempt; true if it is accepted
+    SUN_HD bool operator()(double al, double& d) const {
+        d = -num / al;
+        return (1.00 - 0.5 * d) > x4 * x4;
+    }
+};
+struct FinalDraws {
+    double a3, sn, cs;
+    FinalDraws() = default;
+    SUN_HD explicit FinalDraws(const uint32_t fin[2]) {
+        a3 = 2.0 * u01(fin[0]) - 1.0;
+        sun_sincos2pi(u01(fin[1]), &sn, &cs);
+    }
+};
+
+// the draws of block `block`, each computed where it is used
+struct KeyDraws {
+    const DrawKey& key;
+    int block;
+    BlockDraws bd;
+    SUN_HD KeyDraws(const DrawKey& k, int b) : key(k), block(b), bd(k, b) {}
+    SUN_HD Attempt first() const { return Attempt(bd.first); }
+    SUN_HD Attempt retry(int k) const {
+        uint32_t w[4];
+        key.words((uint32_t)block * kBlockCounters + (uint32_t)k, w);
+        return Attempt(w);
+    }
+    SUN_HD FinalDraws fin() const { return FinalDraws(bd.fin); }
+};
+
 // SU(2) element a = (a0,a1,a2,a3) with a0 ~ sqrt(1-a0^2) exp(al*a0): the MILC
 // Kennedy-Pendleton generator with the Creutz fallback for al <= 2, restating
 // device_PHB_OVR.h:162-223 (including the 1e-10 guard and the 20-try caps), with the
-// uniforms of block `block` (bd: its first attempt and final words; retries from
-// key).  The reference's double literals make this arithmetic double even for
-// Real=float; here it is double for every storage precision but the FP32 SU(3) path.
-// Its log, exp and sin/cos of 2 pi u are sun_libm.h's, which give the same bits on
-// the host and the device.
-SUN_HD void generate_su2_milc(double al, const DrawKey& key, int block, const BlockDraws& bd, double a[4]) {
+// uniforms of block `block`: draws.first(), retry(k) and fin().  The reference's double literals make this arithmetic double
+// even for Real=float; here it is double for every storage precision but the FP32 SU(3)
+// path.  Its log, exp and sin/cos of 2 pi u are sun_libm.h's, which give the same bits
+// on the host and the device.
+template <typename DRAWS>
+SUN_HD void generate_su2_milc(double al, const DrawKey& key, int block, const DRAWS& draws, double a[4]) {
     double xr1, xr2, xr3, xr4, d, r;
     double a0 = 0.0;
-    xr1 = u01(bd.first[0]);
-    xr1 = sun_log(xr1 + 1.e-10);
-    xr2 = u01(bd.first[1]);
-    xr2 = sun_log(xr2 + 1.e-10);
-    xr3 = u01(bd.first[2]);
-    xr4 = u01(bd.first[3]);
-    xr3 = sun_cos2pi(xr3);
-    d = -(xr2 + xr1 * xr3 * xr3) / al;
-    bool accepted = (1.00 - 0.5 * d) > xr4 * xr4;
+    bool accepted = draws.first()(al, d);
     const uint32_t cbase = (uint32_t)block * kBlockCounters;
     if (!accepted && al > 2.0) {
-        for (int k = 1; k <= 20; k++) {
-            uint32_t w[4];
-            key.words(cbase + (uint32_t)k, w);
-            xr1 = u01(w[0]);
-            xr1 = sun_log(xr1 + 1.e-10);
-            xr2 = u01(w[1]);
-            xr2 = sun_log(xr2 + 1.e-10);
-            xr3 = u01(w[2]);
-            xr4 = u01(w[3]);
-            xr3 = sun_cos2pi(xr3);
-            d = -(xr2 + xr1 * xr3 * xr3) / al;
-            if ((1.00 - 0.5 * d) > xr4 * xr4) break;
-        }
+        for (int k = 1; k <= 20; k++)
+            if (draws.retry(k)(al, d)) break;
     }
     if (!accepted && al <= 2.0) {
         xr3 = sun_exp(-2.0 * al);
@@ -229,14 +257,13 @@ SUN_HD void generate_su2_milc(double al, const DrawKey& key, int block, const Bl
     xr3 = 1.0 - a[0] * a[0];
     xr3 = fabs(xr3);
     r = sqrt(xr3);
-    a[3] = (2.0 * u01(bd.fin[0]) - 1.0) * r;
+    const FinalDraws f = draws.fin();
+    a[3] = f.a3 * r;
     xr1 = xr3 - a[3] * a[3];
     xr1 = fabs(xr1);
     xr1 = sqrt(xr1);
-    double sn, cs;
-    sun_sincos2pi(u01(bd.fin[1]), &sn, &cs);
-    a[1] = xr1 * cs;
-    a[2] = xr1 * sn;
+    a[1] = xr1 * f.cs;
+    a[2] = xr1 * f.sn;
 }
 
 // The same generator evaluated in FP32 (uniforms rounded to float), used by the
