@@ -51,12 +51,17 @@ void release(sun_wlop* h) {
 }
 
 // Few T: multiplying every link out takes less time than moving the operators along time
-// lines (us per correlator, multiplied out / moved: FP64 A0, 16^3 x 32: 196 / 273 for two T,
-// 369 / 276 for four; 8^3 x 16: 44 / 61 and 53 / 61; FP32 A0, 16^4: 144 / 198 for six, 218 / 205
-// for nine; FP64 33 family, 16^3 x 32: 429 / 662 for one T, then more than moved).
-bool wlop_direct(int nop, int T1, int precision) {
-    if (nop > 16) return T1 <= 1;
-    return T1 <= (precision == SUN_PREC_F64 ? 3 : 8);
+// lines.  us per correlator, multiplied out / moved, around the rule's line:
+//   A0 FP64   16^3 x 32 SU(3) 225 / 258 for three T, 304 / 263 for four; 8^3 x 16 62 / 66 for six,
+//             71 / 66 for seven; SU(4) 12^3 x 24 199 / 246 for two, 293 / 245 for three
+//   A0 FP32   16^4 140 / 143 for seven, 158 / 142 for eight (8^3 x 16 72 / 76, 16^3 x 32 279 / 240)
+//   33 FP64   16^3 x 32 368 / 546 for one, 775 / 553 for two
+//   33 FP32   16^3 x 32 491 / 617 for four, 630 / 616 for five; SU(4) 12^3 x 24 314 / 302 for two
+bool wlop_direct(int nop, int T1, const sun_lattice* lat) {
+    const bool f64 = lat->d.precision == SUN_PREC_F64;
+    if (nop > 16) return T1 <= (f64 || lat->d.nc > 3 ? 1 : 4);
+    if (f64) return T1 <= (lat->d.nc > 3 ? 2 : 3) + std::min(3, 30000 / lat->g.V);
+    return T1 <= 7;
 }
 
 int check_radius(const sun_wlop* h, int r, int mu, const char* what) {
@@ -88,7 +93,7 @@ extern "C" int sun_wlop_create(sun_lattice* lat, int family, int tmax, sun_wlop*
     h->stride = (size_t)g.V * h->lb;
     h->nb = monitor_blocks(g);
     h->rows = wlop_corr_blocks(g);
-    h->direct = wlop_direct(nop, tmax + 1, lat->d.precision);
+    h->direct = wlop_direct(nop, tmax + 1, lat);
     const size_t nout = (size_t)nop * nop * (tmax + 1);
     const size_t npart = nout * (size_t)std::max(h->nb, h->rows);
     const size_t line = (size_t)2 * lat->d.nc * lat->d.nc * sizeof(double), vs = (size_t)g.str[3];

@@ -96,3 +96,19 @@ def test_operator_loops_of_ragged_volumes(ctx, oracle, family, dims, rmax, nc, s
         got = lat.wilson_loops_ops(rmax, 5, family)
     want = oracle.wilson_loops_ops(U, dims, rmax, 5, family)
     assert np.abs(got - want).max() <= (1e-12 if prec == 8 else 2e-5)
+
+
+# the numbers of T at which the matrix-core correlator takes one more column of tiles or workgroup
+@pytest.mark.parametrize("tmax", [5, 6, 8, 9, 11, 12, 14, 15, 17, 18, 20])
+@pytest.mark.parametrize("nc,prec,family,kind", [(3, 8, 0, "unitary"), (3, 8, 0, "scattered"), (2, 4, 0, "scattered"),
+                                                 (3, 8, 1, "unitary"), (3, 4, 1, "scattered"), (4, 8, 1, "scattered")])
+def test_correlator_tiles(ctx, oracle, nc, prec, family, kind, tmax):
+    dims, r, mu = (2, 4, 2, 22), 1, 1
+    with sun_amd.Lattice(ctx, nc, dims, BETAS[nc], 18, prec) as lat:
+        U = field(lat, oracle, nc, dims, kind)
+        with sun_amd.WilsonLoopOps(lat, family, tmax) as ops:
+            ops.fields(r, mu)
+            ops.correlate(r, mu)
+            got = ops.read()
+    want = oracle.wlop_correlate(U, dims, oracle.wlop_fields(U, dims, family, r, mu), r, mu, tmax)
+    assert np.abs(got - want).max() <= BAR[prec] * np.abs(want).max()
