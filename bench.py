@@ -32,6 +32,7 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 PEAK_HBM_GBS = 8000.0
+PEAK_F64_TFS = 78.6  # FP64 matrix
 DIMS = (32, 32, 32, 32)
 BETA = 6.0
 
@@ -577,13 +578,12 @@ def operator_loops_leg(sun_amd, ctx, stream, calibrate=False):
     """Operator-basis Wilson loops on a 32^4 SU(3) FP64 18-real field (the
     reference's A0 measurement, test.cpp:255-298: Sigma_g_plus(12, 16), r = 2..12,
     the three spatial directions; the 33 family's operator field and correlator at
-    r = 12).  Roofline of the correlator launch: algorithmic bytes per launch = V x
-    144 B x (nop bottom operators + nop (T + 1) top operators + 2 T temporal links)
-    plus its FP64 partials, over the launch time measured with HIP events on its
-    stream.  calibrate: two plain copies of the 604 MB link field first (the size
+    r = 12).  Roofline of the correlator: FP64 operations of the traces, V nop^2 (T + 1)
+    Frobenius products of 18 reals, over the time of one correlator (its time lines,
+    matrix-core kernel and finalize) measured with HIP events on its stream.  calibrate: two plain copies of the 604 MB link field first (the size
     reference for counter passes)."""
     V = int(np.prod(DIMS))
-    lb, T = 144, 16
+    T = 16
     out = {"lattice": list(DIMS), "precision": "f64", "storage": 18, "rmax": 12, "tmax": T}
     with sun_amd.Lattice(ctx, 3, DIMS, BETA, 18, 8) as lat:
         lat.hot_start(21, stream)
@@ -617,13 +617,12 @@ def operator_loops_leg(sun_amd, ctx, stream, calibrate=False):
                 tm.stop(stream)
                 c_ms = tm.ms() / 5
                 tm.close()
-                nb = (V + 255) // 256
-                alg = V * lb * (nop + nop * (T + 1) + 2 * T) + nop * nop * (T + 1) * nb * 8
-                gbs = alg / (c_ms * 1e-3) / 1e9
+                alg = V * nop * nop * (T + 1) * 36
+                tfs = alg / (c_ms * 1e-3) / 1e12
                 out[name] = {"nop": nop, "fields_ms_r12": f_ms, "correlate_ms_r12": c_ms,
-                             "correlate_roofline": {"bound": "hbm", "achieved": gbs, "peak": PEAK_HBM_GBS,
-                                                    "unit": "GB/s", "frac": gbs / PEAK_HBM_GBS,
-                                                    "alg_bytes_per_launch": alg}}
+                             "correlate_roofline": {"bound": "mfma_f64", "achieved": tfs, "peak": PEAK_F64_TFS,
+                                                    "unit": "TFLOP/s", "frac": tfs / PEAK_F64_TFS,
+                                                    "alg_flops_per_correlator": alg}}
     return out
 
 
