@@ -217,8 +217,8 @@ int sun_wilson_loops(sun_lattice *lat, int rmax, int tmax, double *out, void *st
 /* sun_wilson_loops without allocating: no counterpart in the reference; for callers
  * that cannot allocate device memory (code under stream/graph capture, serving loops,
  * harnesses that forbid hipMalloc).  Same kernels and results (bit for bit), but the
- * Wilson-line field and the partial sums live in a fixed 32 MiB device array (one per
- * GPU, held until the process ends) and W(r, T) goes to DEVICE memory dev_out (16-byte
+ * time lines or the Wilson-line field and the partial sums live in a fixed 32 MiB device
+ * array (one per GPU, held until the process ends) and W(r, T) goes to DEVICE memory dev_out (16-byte
  * aligned, 2 (rmax+1)(tmax+1) doubles, same layout as out), asynchronously on the
  * stream.  Needs 3V x 2N^2 x precision bytes for the line field plus 48 (tmax+1)
  * ceil(V/256) for the partials: SU(3) up to 16^4 in FP64 and 16^3x32 in FP32;

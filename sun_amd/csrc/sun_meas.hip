@@ -178,6 +178,22 @@ WlPlanes wl_planes(const sun_lattice* lat, int tmax) {
     return w;
 }
 
+// of sun_wilson_loops_noalloc: the line field and the partial sums of the multiplied-out loops
+size_t wl_line_bytes(const sun_lattice* lat) {
+    return (3 * (size_t)lat->g.V * 2 * lat->d.nc * lat->d.nc * (size_t)lat->d.precision + 255) & ~(size_t)255;
+}
+size_t wl_part_bytes(const sun_lattice* lat, int tmax) {
+    return (size_t)3 * (tmax + 1) * monitor_blocks(lat->g) * sizeof(double2);
+}
+
+// Both entry points take the same route, for the same bits: by planes where they fit LDS, except
+// sizes that sun_wilson_loops_noalloc accepts but whose time lines its array does not hold
+bool wl_takes_planes(const sun_lattice* lat, const WlPlanes& w, int tmax) {
+    if (!w.fits()) return false;
+    if (wl_line_bytes(lat) + wl_part_bytes(lat, tmax) > kNoAllocScratchBytes) return true;
+    return w.lines + w.per_radius <= kNoAllocScratchBytes && line_blocks(lat->g) * sizeof(int) <= kNoAllocStateBytes;
+}
+
 double wl_scale(const sun_lattice* lat) { return 1.0 / (3.0 * lat->d.nc * (double)lat->g.V); }  // wilsonloop.cu:512
 
 // Condition number up to which time lines are inverted (FP64 arithmetic), FP32 and FP64
@@ -228,7 +244,7 @@ static int sun_wilson_loops_body(sun_lattice* lat, int rmax, int tmax, double* o
     std::vector<double2> h(nres);
     const WlPlanes w = wl_planes(lat, tmax);
     bool done = false;
-    if (w.fits()) {
+    if (wl_takes_planes(lat, w, tmax)) {
         constexpr size_t kPartBytes = size_t(64) << 20;  // of partial sums at a time
         const size_t part = std::max(w.per_radius, std::min(w.per_radius * (rmax + 1), kPartBytes));
         std::vector<int> st(line_blocks(g));
@@ -281,9 +297,7 @@ extern "C" int sun_wilson_loops_noalloc(sun_lattice* lat, int rmax, int tmax, do
     if (!lat->ctx->scratch) return fail(SUN_ERR_STATE, "sun_wilson_loops_noalloc: no scratch array on this device");
     const size_t full = (size_t)2 * lat->d.nc * lat->d.nc * (size_t)lat->d.precision;  // 18-real record
     const size_t nline = 3 * (size_t)g.V;
-    const int nb = monitor_blocks(g);
-    const size_t line_bytes = (nline * full + 255) & ~(size_t)255;
-    const size_t part_bytes = (size_t)3 * (tmax + 1) * nb * sizeof(double2);
+    const size_t line_bytes = wl_line_bytes(lat), part_bytes = wl_part_bytes(lat, tmax);
     if (line_bytes + part_bytes > kNoAllocScratchBytes)
         return fail(SUN_ERR_BUDGET,
                     "sun_wilson_loops_noalloc: needs %zu bytes of scratch (line field %zu + partials %zu), the "
@@ -295,8 +309,7 @@ extern "C" int sun_wilson_loops_noalloc(sun_lattice* lat, int rmax, int tmax, do
     double2* res = reinterpret_cast<double2*>(dev_out);
     const WlPlanes w = wl_planes(lat, tmax);
     int* state = nullptr;
-    if (w.fits() && w.lines + w.per_radius <= kNoAllocScratchBytes &&
-        line_blocks(g) * sizeof(int) <= kNoAllocStateBytes) {
+    if (wl_takes_planes(lat, w, tmax)) {
         state = reinterpret_cast<int*>(base + kNoAllocScratchBytes);
         SUN_TRY(wl_by_planes(lat, w, rmax, tmax, reinterpret_cast<double*>(base),
                              reinterpret_cast<double2*>(base + w.lines), kNoAllocScratchBytes - w.lines, state, res, s));
