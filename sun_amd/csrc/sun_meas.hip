@@ -196,14 +196,14 @@ bool wl_takes_planes(const sun_lattice* lat, const WlPlanes& w, int tmax) {
 
 double wl_scale(const sun_lattice* lat) { return 1.0 / (3.0 * lat->d.nc * (double)lat->g.V); }  // wilsonloop.cu:512
 
-// Condition number up to which time lines are inverted (FP64 arithmetic), FP32 and FP64
-// lattices: rounding errors grow by at most its square
-constexpr double kWlCond[2] = {1e3, 1e2};
+// Time lines that are inverted (FP64 arithmetic), FP32 and FP64 lattices: rounding errors
+// grow by at most the square of the condition number
+constexpr LineLimits kWlLines[2] = {{1e3, 1e60}, {1e2, 1e60}};
 
 int wl_by_planes(sun_lattice* lat, const WlPlanes& w, int rmax, int tmax, double* P, double2* part, size_t part_bytes,
                  int* state, double2* res, hipStream_t s) {
     const Geom& g = lat->g;
-    HIP_TRY(lat->ops->time_lines(lat->f, g, g.X[3] + 1, true, kWlCond[lat->d.precision == SUN_PREC_F64], P, nullptr,
+    HIP_TRY(lat->ops->time_lines(lat->f, g, g.X[3] + 1, true, kWlLines[lat->d.precision == SUN_PREC_F64], P, nullptr,
                                  state, s));
     const int group = (int)std::min<size_t>((size_t)rmax + 1, part_bytes / w.per_radius);
     const int nb[3] = {w.ps[0].blocks, w.ps[1].blocks, 0};

@@ -159,6 +159,11 @@ inline PlaneShape plane_shape(const Geom& g, int T1, int bytes) {
     return p;
 }
 
+// What time lines may be inverted (sun_transport.inc): condition number and norms
+struct LineLimits {
+    double cond, range;
+};
+
 struct OpsTable {
     int nc, storage, real_bytes;
     // one (parity, mu) heatbath (hb=true) or overrelaxation launch
@@ -228,9 +233,9 @@ struct OpsTable {
     // time lines of every spatial site: P of `next` times (element by element where
     // `planes`), inverses Q (may be null) of X3
     // times, FP64 N x N matrices; state[line_blocks(geom)]: per block whether its lines are
-    // unitary (0), have condition numbers up to cond (1) or not (kLinesBad)
-    hipError_t (*time_lines)(const Field& f, const Geom&, int next, bool planes, double cond, double* P, double* Q, int* state,
-                             hipStream_t);
+    // unitary (0), within the limits (1) or not (kLinesBad)
+    hipError_t (*time_lines)(const Field& f, const Geom&, int next, bool planes, const LineLimits& lim, double* P, double* Q,
+                             int* state, hipStream_t);
     // the correlator of every slot pair; time lines of next = X3 + tmax times.  Partials:
     // [wlop_corr_blocks][T][i][j], or, where a state is kLinesBad,
     // [(i nop + j)(tmax + 1) + T][monitor_blocks]; state null: the latter, without lines

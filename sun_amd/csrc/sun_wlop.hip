@@ -152,15 +152,17 @@ extern "C" int sun_wlop_fields(sun_wlop* h, int r, int mu, void* stream) {
     return fields(h, r, mu, true, s);
 }
 
-// Condition number up to which time lines are inverted, FP32 and FP64 lattices (whose X and
-// Y are formed in FP32 and FP64): rounding errors grow by at most its square, to about 1e-12
-// of a loop in FP64 and, in FP32, to what a dozen products of FP32 links carry.
-constexpr double kLineCond[2] = {4.0, 100.0};
+// Time lines that are inverted, FP32 and FP64 lattices (whose X and Y are formed in FP32 and
+// FP64): rounding errors grow by at most the square of the condition number, to about 1e-12
+// of a loop in FP64 and, in FP32, to what a dozen products of FP32 links carry.  X and Y stay
+// within the range times the operators (Y within its square past the lattice's end), far
+// from the limits of FP32.
+constexpr LineLimits kLines[2] = {{4.0, 1e8}, {100.0, 1e60}};
 
 // the time lines of the lattice's present temporal links
 static int time_lines(sun_wlop* h, hipStream_t s) {
     if (h->direct) return SUN_OK;
-    HIP_TRY(h->lat->ops->time_lines(h->lat->f, h->lat->g, h->lat->g.X[3] + h->tmax, false, kLineCond[h->lat->d.precision == SUN_PREC_F64], h->lines, h->inverses, h->state, s));
+    HIP_TRY(h->lat->ops->time_lines(h->lat->f, h->lat->g, h->lat->g.X[3] + h->tmax, false, kLines[h->lat->d.precision == SUN_PREC_F64], h->lines, h->inverses, h->state, s));
     return SUN_OK;
 }
 
