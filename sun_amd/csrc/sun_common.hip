@@ -109,7 +109,7 @@ __global__ void __launch_bounds__(kReduceBlock) k_finalize_iteration(const doubl
     }
 }
 
-__global__ void __launch_bounds__(kReduceBlock) k_wl_finalize(const double2* partials, int nb_unitary, int nb_general,
+__global__ void __launch_bounds__(kReduceBlock) k_wl_finalize(const double2* partials, int nb_near, int nb_general,
                                                               int nb_bad, int tmax, double scale, const int* state,
                                                               int nstate, double2* out) {
     int nb = nb_bad;
@@ -121,7 +121,7 @@ __global__ void __launch_bounds__(kReduceBlock) k_wl_finalize(const double2* par
         }
         bad = __syncthreads_or(bad);
         general = __syncthreads_or(general);
-        nb = bad ? nb_bad : general ? nb_general : nb_unitary;
+        nb = bad ? nb_bad : general ? nb_general : nb_near;
     }
     if (!nb) return;
     const int T = blockIdx.x;

@@ -162,8 +162,8 @@ extern "C" int sun_multihit_ext(sun_lattice* in, sun_lattice* out, uint64_t seed
 namespace {
 
 struct WlPlanes {
-    PlaneShape ps[2];        // unitary time lines, others
-    size_t lines, per_radius;  // bytes
+    PlaneShape ps[2];  // time lines near to unitary, others
+    size_t off, lines, per_radius;  // bytes: of the lines, with what they are off unitary, of the sums of a radius
     bool fits() const { return ps[0].sites && ps[1].sites; }
 };
 
@@ -173,7 +173,8 @@ WlPlanes wl_planes(const sun_lattice* lat, int tmax) {
     WlPlanes w;
     w.ps[0] = plane_shape(g, tmax + 1, (int)(reals * lat->d.precision));
     w.ps[1] = plane_shape(g, tmax + 1, (int)(reals * sizeof(double)));
-    w.lines = ((size_t)g.str[3] * (g.X[3] + 1) * reals * sizeof(double) + 255) & ~(size_t)255;
+    w.off = ((size_t)g.str[3] * (g.X[3] + 1) * reals * sizeof(double) + 255) & ~(size_t)255;
+    w.lines = w.off + (((size_t)g.V * (reals / 2 + 3) * lat->d.precision + 255) & ~(size_t)255);
     w.per_radius = (size_t)3 * (tmax + 1) * std::max(w.ps[0].blocks, w.ps[1].blocks) * sizeof(double2);
     return w;
 }
@@ -203,13 +204,13 @@ constexpr LineLimits kWlLines[2] = {{1e3, 1e60}, {1e2, 1e60}};
 int wl_by_planes(sun_lattice* lat, const WlPlanes& w, int rmax, int tmax, double* P, double2* part, size_t part_bytes,
                  int* state, double2* res, hipStream_t s) {
     const Geom& g = lat->g;
-    HIP_TRY(lat->ops->time_lines(lat->f, g, g.X[3] + 1, true, kWlLines[lat->d.precision == SUN_PREC_F64], P, nullptr,
-                                 state, s));
+    void* E = (char*)P + w.off;
+    HIP_TRY(lat->ops->time_lines(lat->f, g, g.X[3] + 1, true, kWlLines[lat->d.precision == SUN_PREC_F64], P, E, state, s));
     const int group = (int)std::min<size_t>((size_t)rmax + 1, part_bytes / w.per_radius);
     const int nb[3] = {w.ps[0].blocks, w.ps[1].blocks, 0};
     for (int r = 0; r <= rmax; r += group) {
         const int hi = std::min(rmax + 1, r + group);
-        HIP_TRY(lat->ops->wl_plane(lat->f, g, r, hi, tmax + 1, g.X[3] + 1, P, state, w.ps, part, s));
+        HIP_TRY(lat->ops->wl_plane(lat->f, g, r, hi, tmax + 1, g.X[3] + 1, P, E, state, w.ps, part, s));
         HIP_TRY(launch_wl_finalize(part, nb, hi - r, tmax, wl_scale(lat), state, line_blocks(g),
                                    res + (size_t)r * (tmax + 1), s));
     }

@@ -215,9 +215,9 @@ struct OpsTable {
                                hipStream_t);
     // Wilson loops of radii [r_lo, r_hi) and T < T1, moved along time lines (planes, next =
     // X3 + 1 times): 3 T1 blocks partials per radius, of the shape's blocks, ps[0] where the
-    // lines are unitary, ps[1] where not; nothing where they are kLinesBad
+    // lines are near to unitary, ps[1] where not; nothing where they are kLinesBad
     hipError_t (*wl_plane)(const Field& f, const Geom&, int r_lo, int r_hi, int T1, int next, const double* P,
-                           const int* state, const PlaneShape ps[2], double2* partials, hipStream_t);
+                           const void* E, const int* state, const PlaneShape ps[2], double2* partials, hipStream_t);
     // the same with the links multiplied out: the Wilson lines of radius r, then its loops;
     // where state is given, only if it is kLinesBad
     hipError_t (*wl_lines)(const Field& f, const Field& lines, const Geom&, int r, const int* state, hipStream_t);
@@ -230,11 +230,11 @@ struct OpsTable {
     // 9 is left as it is)
     hipError_t (*wlop_fields)(const Field& f, char* ops, char* aux, size_t stride, const Geom&, int family, int r,
                               int mu, double rt8, bool exact, hipStream_t);
-    // time lines of every spatial site: P of `next` times (element by element where
-    // `planes`), inverses Q (may be null) of X3
-    // times, FP64 N x N matrices; state[line_blocks(geom)]: per block whether its lines are
-    // unitary (0), within the limits (1) or not (kLinesBad)
-    hipError_t (*time_lines)(const Field& f, const Geom&, int next, bool planes, const LineLimits& lim, double* P, double* Q,
+    // time lines of every spatial site: P of `next` times, inverses Q of X3 times, FP64 N x N
+    // matrices; where `planes`, P element by element and Q the N^2 reals of the links'
+    // precision by which P P^+ is off 1; state[line_blocks(geom)]: per block whether its lines
+    // are near to unitary (0), within the limits (1) or not (kLinesBad)
+    hipError_t (*time_lines)(const Field& f, const Geom&, int next, bool planes, const LineLimits& lim, double* P, void* Q,
                              int* state, hipStream_t);
     // the correlator of every slot pair; time lines of next = X3 + tmax times.  Partials:
     // [wlop_corr_blocks][T][i][j], or, where a state is kLinesBad,

@@ -30,7 +30,7 @@ struct sun_wlop {
     bool direct = false;    // few T: without time lines
     double* lines = nullptr;   // time lines: X3 + tmax times of every spatial site
     double* inverses = nullptr;  // their inverses, X3 times
-    int* state = nullptr;   // per block of lines, whether they are unitary or can be inverted
+    int* state = nullptr;   // per block of lines, what they allow
     double* acc = nullptr;  // nop^2 (tmax + 1), (i nop + j)(tmax + 1) + T
     int r = -1, mu = -1;    // radius and direction of the current operator field
 };
