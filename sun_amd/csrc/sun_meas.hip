@@ -197,9 +197,12 @@ bool wl_takes_planes(const sun_lattice* lat, const WlPlanes& w, int tmax) {
 
 double wl_scale(const sun_lattice* lat) { return 1.0 / (3.0 * lat->d.nc * (double)lat->g.V); }  // wilsonloop.cu:512
 
-// Time lines that are inverted (FP64 arithmetic), FP32 and FP64 lattices: rounding errors
-// grow by at most the square of the condition number
-constexpr LineLimits kWlLines[2] = {{1e3, 1e60}, {1e2, 1e60}};
+// Time lines that are inverted (FP64 arithmetic), FP32 and FP64 lattices.  Rounding errors
+// grow with the square of the condition number: FP32 lattices have that to spare (1e-10 at
+// 1e3).  FP64 ones have not: against multiplied-out links the errors of single loops (SU(3),
+// 32 times) are 1.1 to 2.4 times as large for T = 16 to 0 up to 1.6, 1.4 to 2.5 times at 2.8, 2
+// to 5 times at 10 and 15 to 41 times at 63, so they take lines up to 2.
+constexpr LineLimits kWlLines[2] = {{1e3, 1e60}, {2.0, 1e60}};
 
 int wl_by_planes(sun_lattice* lat, const WlPlanes& w, int rmax, int tmax, double* P, double2* part, size_t part_bytes,
                  int* state, double2* res, hipStream_t s) {

@@ -153,11 +153,11 @@ extern "C" int sun_wlop_fields(sun_wlop* h, int r, int mu, void* stream) {
 }
 
 // Time lines that are inverted, FP32 and FP64 lattices (whose X and Y are formed in FP32 and
-// FP64): rounding errors grow by at most the square of the condition number, to about 1e-12
-// of a loop in FP64 and, in FP32, to what a dozen products of FP32 links carry.  X and Y stay
-// within the range times the operators (Y within its square past the lattice's end), far
-// from the limits of FP32.
-constexpr LineLimits kLines[2] = {{4.0, 1e8}, {100.0, 1e60}};
+// FP64): up to the condition numbers at which rounding errors, which grow with their square,
+// stay those of the links multiplied out (measured for Wilson loops, sun_meas.hip).  X and Y
+// stay within the range times the operators (Y within its square past the lattice's end),
+// far from the limits of FP32.
+constexpr LineLimits kLines[2] = {{1.2, 1e8}, {2.0, 1e60}};
 
 // the time lines of the lattice's present temporal links
 static int time_lines(sun_wlop* h, hipStream_t s) {

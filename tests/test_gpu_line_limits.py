@@ -8,7 +8,11 @@ And lines that are unitary but for the rounding of their links, which leans to o
 many updates without reunitarisation: a loop takes the T links that it has, not the X3 of its
 lines.  The errors of single loops (a few roundings, 1e-16 and 6e-8) average out over the loops of
 a volume, so the bars are a few roundings: FP64 4e-15 of the loops and 6e-15 of the largest
-correlator, FP32 4e-8 and 1e-7.  The deviations of whole lines are 3e-14 and 5e-7."""
+correlator, FP32 4e-8 and 1e-7.  The deviations of whole lines are 3e-14 and 5e-7.
+
+And lines that a single time slice makes badly conditioned: through the inverses of such lines the
+loops that do not touch the slice lose the condition number's square, 2e4 roundings in FP64 and 60
+in FP32; multiplied out they have a few.  Bars: 1e-14 and 6e-8 of the largest correlator of each T."""
 import numpy as np
 import pytest
 
@@ -94,3 +98,32 @@ def test_links_that_lean_to_one_side(ctx, oracle, nc, prec):
         fields = [oracle.wlop_fields(U, dims, family, 2, mu) for mu in range(3)]
         want = correlators(U, dims, fields, 2, 8)
         assert np.abs(ops[family][0] - want).max() <= (6e-15 if prec == 8 else 1e-7) * np.abs(want).max()
+
+
+def stretched(oracle, nc, dims, condition):
+    """the links of the first time slice times a matrix of |m| |m^-1| / N = condition (not a diagonal one: what
+    that costs, row by row, its inverse gives back)"""
+    U = thermalised(oracle, nc, dims, 18).copy()
+    a = np.roots([1, -(nc * condition - (nc - 2)), 1]).real.max() ** 0.5  # (a^2 + 1/a^2 + N - 2) / N
+    first = np.arange(U.shape[1]) % (U.shape[1] // 2) < U.shape[1] // 2 // dims[3]
+    rng = np.random.default_rng(1)
+    left, right = (np.linalg.qr(rng.normal(size=(nc, nc)) + 1j * rng.normal(size=(nc, nc)))[0] for _ in range(2))
+    U[3, first] = left @ np.diag([a, 1 / a, 1, 1][:nc]) @ right @ U[3, first]
+    return U
+
+
+@pytest.mark.parametrize("nc,prec", [(2, 8), (3, 8), (2, 4), (3, 4)])
+def test_badly_conditioned_lines(ctx, oracle, nc, prec):
+    dims, tmax = (2, 2, 2, 16), 8
+    U = stretched(oracle, nc, dims, 90 if prec == 8 else 3.8)
+    with sun_amd.Lattice(ctx, nc, dims, BETAS[nc], 18, prec) as lat:
+        lat.from_host(U)
+        U = lat.to_host()
+        got = lat.wilson_loops(2, tmax).real
+        ops = [lat.wilson_loops_ops(2, tmax, family)[0] for family in (0, 1)]
+    bar = 1e-14 if prec == 8 else 6e-8
+    want = np.array([correlators(U, dims, lines(oracle, U, dims, r), r, tmax)[0] for r in range(3)])
+    assert (np.abs(got - want).max(0) <= bar * np.abs(want).max(0)).all()
+    for family in (0, 1):
+        want = correlators(U, dims, [oracle.wlop_fields(U, dims, family, 2, mu) for mu in range(3)], 2, tmax)
+        assert (np.abs(ops[family] - want).max(0) <= bar * np.abs(want).max(0)).all()
