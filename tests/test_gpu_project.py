@@ -46,3 +46,15 @@ def test_projection_of_zero(ctx, nc, prec):
         lat.ape_smear(0.2, 1, 10)
         got = lat.to_host()[:3]
     assert np.array_equal(got, np.broadcast_to(np.eye(nc) if nc == 3 else np.zeros((nc, nc)), got.shape))
+
+
+@pytest.mark.parametrize("nc", [2, 3, 4])
+def test_fp32_projection_keeps_the_norm(ctx, nc):
+    """Thirty and more reciprocal roots, one after another, none of them leaning to one side: the norm of a
+    projected link is off by some 1e-6 at most, its mean over V x 3 links (2304) by a fiftieth of that, 2e-8
+    (the native instruction alone is 7e-9 too small, links 4e-7 after ten hits)."""
+    with sun_amd.Lattice(ctx, nc, DIMS, 6.0, 18, 4) as lat:
+        lat.from_host(links(nc))
+        lat.ape_smear(0.2, 1, 20)
+        u = lat.to_host()[:3]
+    assert abs((np.abs(u) ** 2).sum((2, 3)).mean() / nc - 1) <= 1e-7
