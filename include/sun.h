@@ -104,7 +104,11 @@ size_t sun_lattice_bytes(const sun_lattice_desc *desc);
  * lds: unused dynamic LDS per workgroup (caps workgroups per CU).  piped: the
  * software-pipelined kernels (FP32 12- and 8-real SU(3)): 1 pipelined by
  * directions (2 waves per SIMD), 2 by half-directions (3 waves).  Replaces the reference's
- * TuneParam override (include/tune.h:36-118); results never depend on it. */
+ * TuneParam override (include/tune.h:36-118); results never depend on it.
+ * Small lattices (FP64 up to 32768 sites; FP64 SU(2), FP64 8-real and FP32 SU(3)
+ * up to 65536) for which no shape is set run a kernel of its own shape instead, which shares
+ * the staple of a link among waves; the autotuner leaves them alone, and get_launch reports
+ * the shape that they would run without it. */
 typedef struct {
     int block, brick[3], lds, piped;
 } sun_launch;

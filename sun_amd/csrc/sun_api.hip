@@ -249,9 +249,10 @@ Field sun::make_field(void* base, size_t nrec, size_t lb) {
 
 // the tuner's launch shapes, or the default ones
 static void set_launches(sun_lattice* L) {
-    Tuner& t = L->ctx->tuner;
-    L->cfg_hb = t.has("heatbath", L->d) ? t.lookup("heatbath", L->d) : default_launch(L->ops, L->g, 0);
-    L->cfg_or = t.has("overrelax", L->d) ? t.lookup("overrelax", L->d) : default_launch(L->ops, L->g, 1);
+    L->cfg_hb = default_launch(L->ops, L->g, 0);
+    L->cfg_or = default_launch(L->ops, L->g, 1);
+    L->ctx->tuner.chosen("heatbath", L->d, L->cfg_hb, &L->cfg_hb);
+    L->ctx->tuner.chosen("overrelax", L->d, L->cfg_or, &L->cfg_or);
 }
 
 static void set_planes(sun_lattice* L) { L->f = make_field(L->buf, 4 * (size_t)L->g.V, link_bytes(&L->d)); }

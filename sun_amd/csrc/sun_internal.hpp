@@ -65,7 +65,9 @@ class Tuner {
    public:
     void load(int mode);
     void save();
-    LaunchCfg lookup(const char* kernel, const sun_lattice_desc& d);
+    // the shape to run instead of dflt: set by the caller, or found by timing among the shapes
+    // (which says nothing about a split default)
+    bool chosen(const char* kernel, const sun_lattice_desc& d, const LaunchCfg& dflt, LaunchCfg* out);
     bool has(const char* kernel, const sun_lattice_desc& d);
     void record(const char* kernel, const sun_lattice_desc& d, const LaunchCfg& c, float ms);
     bool enabled() const { return mode_ != 0; }

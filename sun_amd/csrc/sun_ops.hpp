@@ -23,6 +23,9 @@ struct LaunchCfg {
     int b1 = -1, b2 = 0, b3 = 0;
     // 1: the software-pipelined overrelaxation kernel (where the variant has one)
     int piped = 0;
+    // the kernel that shares a link's staple among waves, whatever the rest says: of small
+    // lattices (default_launch) for which nobody has set a shape
+    bool split = false;
 };
 
 // Brick mapping of workgroups to lattice sites.  The sites of one parity form rows
@@ -244,6 +247,7 @@ struct OpsTable {
     int max_block;   // largest workgroup the update kernels are compiled for
     int has_piped;   // the variant has the software-pipelined overrelaxation kernel
     int piped_max_block;
+    int split_groups;  // workgroups of 64 links up to which the shared-staple kernel is the faster one
 };
 
 // The launch shape of a lattice's updates unless the tuner or the caller has one (kernel 0
@@ -266,6 +270,7 @@ inline LaunchCfg default_launch(const OpsTable* ops, const Geom& g, int kernel) 
     LaunchCfg c;
     const bool f64 = ops->real_bytes == 8, full = ops->storage == 18, hb = kernel == 0;
     const int rows = g.X[0] / 2;
+    c.split = (g.half + 63) / 64 <= ops->split_groups;
     const bool large = g.V > (1 << 18);
     if (ops->has_piped && (ops->storage == 12 || !hb || g.V <= (1 << 19))) c.piped = 2;
     if (!large || (f64 && !full) || (ops->storage == 8 && c.piped)) c.block = 64;

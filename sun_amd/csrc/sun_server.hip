@@ -283,11 +283,9 @@ int rebuild_tables(Group* g) {
                 // the context's shape for this lattice description when it has one
                 // (autotuner cache or sun_ctx_set_launch), else the batch defaults
                 const char* name = k == 0 ? "heatbath" : "overrelax";
-                if (L->ctx->tuner.has(name, L->d)) {
-                    m.cfg[k] = L->ctx->tuner.lookup(name, L->d);
-                    continue;
-                }
                 LaunchCfg c;
+                c.split = default_launch(L->ops, L->g, k).split;
+                if (L->ctx->tuner.chosen(name, L->d, c, &m.cfg[k])) continue;
                 c.block = 256;
                 c.lds = g->lds[k];
                 c.piped = g->piped[k];

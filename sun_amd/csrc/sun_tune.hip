@@ -99,11 +99,12 @@ void Tuner::save() {
     dirty_ = false;
 }
 
-LaunchCfg Tuner::lookup(const char* kernel, const sun_lattice_desc& d) {
+bool Tuner::chosen(const char* kernel, const sun_lattice_desc& d, const LaunchCfg& dflt, LaunchCfg* out) {
     std::lock_guard<std::mutex> lk(mu_);
     auto it = cache_.find(key(kernel, d));
-    if (it != cache_.end()) return it->second.first;
-    return LaunchCfg();
+    if (it == cache_.end() || (dflt.split && it->second.second > 0.f)) return false;
+    *out = it->second.first;
+    return true;
 }
 
 bool Tuner::has(const char* kernel, const sun_lattice_desc& d) {
@@ -122,6 +123,10 @@ void Tuner::record(const char* kernel, const sun_lattice_desc& d, const LaunchCf
 int tune_lattice(sun_lattice* lat, hipStream_t s) {
     sun_ctx* ctx = lat->ctx;
     if (!ctx->tuner.enabled() || lat->tuned) return SUN_OK;
+    if (lat->cfg_hb.split && lat->cfg_or.split) {  // no shape to choose
+        lat->tuned = true;
+        return SUN_OK;
+    }
     void* backup = nullptr;
     HIP_TRY(ctx->spare.allocate(&backup, lat->bytes));
     hipEvent_t e0 = nullptr, e1 = nullptr;
@@ -146,6 +151,7 @@ int tune_lattice(sun_lattice* lat, hipStream_t s) {
     float best_k_ms[2] = {1e30f, 1e30f};
     for (int k = 0; k < 2 && e == hipSuccess; k++) {
         const bool hb = k == 0;
+        if ((hb ? lat->cfg_hb : lat->cfg_or).split) continue;
         // coarse pass: every (kernel, shape, LDS cap) candidate, 8 launches each; piped
         // 0 plain kernel, 1 pipelined by directions, 2 pipelined by half-directions
         std::vector<std::pair<LaunchCfg, float>> cands;
@@ -195,10 +201,12 @@ int tune_lattice(sun_lattice* lat, hipStream_t s) {
         best_k_ms[k] = total[win];
     }
     if (e == hipSuccess) {
-        lat->cfg_hb = best_k[0];
-        lat->cfg_or = best_k[1];
-        ctx->tuner.record("heatbath", lat->d, best_k[0], best_k_ms[0]);
-        ctx->tuner.record("overrelax", lat->d, best_k[1], best_k_ms[1]);
+        for (int k = 0; k < 2; k++) {
+            LaunchCfg& cfg = k == 0 ? lat->cfg_hb : lat->cfg_or;
+            if (cfg.split) continue;
+            cfg = best_k[k];
+            ctx->tuner.record(k == 0 ? "heatbath" : "overrelax", lat->d, best_k[k], best_k_ms[k]);
+        }
     }
     if (e == hipSuccess) e = hipMemcpyAsync(lat->buf, backup, lat->bytes, hipMemcpyDeviceToDevice, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
