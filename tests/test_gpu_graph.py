@@ -43,3 +43,46 @@ def test_long_batch_calls_replay_a_graph(ctx):
             lat.close()
     assert np.array_equal(out[0][0], out[1][0])
     assert all(np.array_equal(a, b) for a, b in zip(out[0][1], out[1][1]))
+
+
+# past the lattices whose updates share staples: bricks, linear order and the pipelined kernels of
+# their default shapes, every storage
+@pytest.mark.parametrize("nc,storage,prec,dims", [(2, 18, 4, (16, 16, 16, 18)), (3, 12, 4, (32, 16, 16, 40)),
+                                                  (3, 8, 4, (16, 16, 16, 18)), (3, 18, 4, (32, 16, 16, 40)),
+                                                  (3, 18, 8, (16, 16, 16, 10)), (3, 12, 8, (16, 16, 16, 10)),
+                                                  (3, 8, 8, (16, 16, 16, 18)), (4, 18, 4, (12, 12, 12, 12))])
+def test_large_lattices_replay_a_graph(ctx, nc, storage, prec, dims):
+    out = []
+    for graph in (False, True):
+        with sun_amd.Lattice(ctx, nc, dims, {2: 2.4, 3: 6.0, 4: 10.8}[nc], storage, prec) as lat:
+            lat.hot_start(3)
+            rows = []
+            for call in range(2):
+                rows.append(lat.generate(7, 24, n_or=1, reunit_every=1 if storage == 8 else 5,
+                                         first_sweep=24 * call, use_graph=graph))
+                lat.overrelax()
+            out.append((rows, lat.to_host()))
+    assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
+
+
+@pytest.mark.parametrize("nc,storage,prec,count", [(3, 12, 4, 24), (3, 8, 4, 36), (4, 18, 4, 10)])
+def test_chunks_on_several_streams_replay_a_graph(ctx, nc, storage, prec, count):
+    """16^4 lattices of 300 MB together: more than three chunks of a third of the 256 MB cache, whose launches
+    the captured iteration forks over the batch's streams"""
+    assert sun_amd.lattice_bytes(nc, (16,) * 4, storage, prec) * count > 3 * (256 << 20) // 3
+    out = []
+    for graph in (False, True):
+        lats = [sun_amd.Lattice(ctx, nc, (16,) * 4, {3: 5.9, 4: 10.8}[nc], storage, prec) for _ in range(count)]
+        for i, lat in enumerate(lats):
+            lat.hot_start(i)
+        batch = sun_amd.Batch(ctx, lats, range(count))
+        rows = []
+        for call in range(2):
+            rows.append(batch.generate(24 * call, 24, n_or=1, use_graph=graph))
+            batch.overrelax()
+        out.append((rows, [lat.plaquette() for lat in lats], lats[0].to_host(), lats[-1].to_host()))
+        batch.close()
+        for lat in lats:
+            lat.close()
+    assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
+    assert np.array_equal(out[0][2], out[1][2]) and np.array_equal(out[0][3], out[1][3])
