@@ -227,12 +227,12 @@ struct OpsTable {
     hipError_t (*wl_loops)(const Field& f, const Field& lines, const Geom&, int r, int tmax, const int* state,
                            double2* partials, hipStream_t);
     // operator-basis Wilson loops: the operator fields of direction mu at radius r
-    // (family 0: 10 slots, 1: 25; slot k, V matrices of 2 N^2 reals one after another, at
-    // ops + k * stride; rt8 = 2 sqrt 2).  exact: FP64 fields with the reference's products one
+    // (family 0: 10 slots, 1: 25; slot k, V matrices of 2 N^2 reals one after another or, where
+    // `planes`, like the links, at ops + k * stride; rt8 = 2 sqrt 2).  exact: FP64 fields with the reference's products one
     // by one, otherwise from shared products (33: in kWlopAuxSlots more slots at aux; A0: slot
     // 9 is left as it is)
     hipError_t (*wlop_fields)(const Field& f, char* ops, char* aux, size_t stride, const Geom&, int family, int r,
-                              int mu, double rt8, bool exact, hipStream_t);
+                              int mu, double rt8, bool exact, bool planes, hipStream_t);
     // time lines of every spatial site: P of `next` times, inverses Q of X3 times, FP64 N x N
     // matrices; where `planes`, P element by element and Q the N^2 reals of the links'
     // precision by which P P^+ is off 1; state[line_blocks(geom)]: per block whether its lines
@@ -344,6 +344,9 @@ inline int partial_slots(const Geom& g) {
 }
 // scratch slots of the 33 family's fields from shared products
 constexpr int kWlopAuxSlots = 14;
+// whether the operator fields of a handle have the links' plane layout (sun_wlop.inc): FP64 and
+// SU(4) fields of A0 handles that multiply every link out (`direct`)
+constexpr bool wlop_planes(bool direct, int nc, bool f64, int nop) { return direct && (f64 || nc == 4) && nop <= 16; }
 // state of time lines that the measurement kernels cannot invert
 constexpr int kLinesBad = 2;
 // workgroups of the time-line kernel (64 spatial sites each)

@@ -28,6 +28,7 @@ struct sun_wlop {
     double* partials = nullptr;
     int nb = 0, rows = 0;   // workgroups of the fallback and of the matrix-core correlator
     bool direct = false;    // few T: without time lines
+    bool planes() const { return wlop_planes(direct, lat->d.nc, lat->d.precision == SUN_PREC_F64, nop); }
     double* lines = nullptr;   // time lines: X3 + tmax times of every spatial site
     double* inverses = nullptr;  // their inverses, X3 times
     int* state = nullptr;   // per block of lines, what they allow
@@ -52,15 +53,18 @@ void release(sun_wlop* h) {
 
 // Few T: multiplying every link out takes less time than moving the operators along time
 // lines.  us per correlator, multiplied out / moved, around the rule's line:
-//   A0 FP64   16^3 x 32 SU(3) 225 / 258 for three T, 304 / 263 for four; 8^3 x 16 62 / 66 for six,
-//             71 / 66 for seven; SU(4) 12^3 x 24 199 / 246 for two, 293 / 245 for three
+//   A0 FP64   SU(3) 8^3 x 16 61 / 64 for seven T, 69 / 64 for eight; 12^4 92 / 90 for seven; 16^3 x
+//             32 264 / 306 for four, 330 / 310 for five; 24^3 x 32 698 / 890 for three, 987 / 889
+//             for four; SU(4) 12^3 x 24 211 / 253 for four, 264 / 254 for five
 //   A0 FP32   16^4 140 / 143 for seven, 158 / 142 for eight (8^3 x 16 72 / 76, 16^3 x 32 279 / 240)
-//   33 FP64   16^3 x 32 368 / 546 for one, 775 / 553 for two
-//   33 FP32   16^3 x 32 491 / 617 for four, 630 / 616 for five; SU(4) 12^3 x 24 314 / 302 for two
+//   33 FP64   16^3 x 32 530 / 619 for two, 795 / 642 for three; 24^3 x 32 1742 / 1820 for two
+//   33 FP32   16^3 x 32 593 / 665 for five, 710 / 665 for six; 24^3 x 32 2230 / 2052 for five; SU(4) 770 / 963 for two, 1150 / 964
+//             for three
 bool wlop_direct(int nop, int T1, const sun_lattice* lat) {
     const bool f64 = lat->d.precision == SUN_PREC_F64;
-    if (nop > 16) return T1 <= (f64 || lat->d.nc > 3 ? 1 : 4);
-    if (f64) return T1 <= (lat->d.nc > 3 ? 2 : 3) + std::min(3, 30000 / lat->g.V);
+    const int V = lat->g.V;
+    if (nop > 16) return T1 <= (f64 || lat->d.nc > 3 ? 2 : V > (1 << 18) ? 4 : 5);
+    if (f64) return T1 <= (V > (1 << 18) ? 3 : V > 25000 ? 4 : V > 10000 ? 6 : 7);
     return T1 <= 7;
 }
 
@@ -138,7 +142,7 @@ extern "C" int sun_wlop_nops(const sun_wlop* h) { return h ? h->nop : 0; }
 static int fields(sun_wlop* h, int r, int mu, bool exact, hipStream_t s) {
     sun_lattice* lat = h->lat;
     HIP_TRY(lat->ops->wlop_fields(lat->f, (char*)h->ops, (char*)h->aux, h->stride, lat->g, h->family, r, mu,
-                                  2.0 * std::sqrt(2.0), exact, s));
+                                  2.0 * std::sqrt(2.0), exact, h->planes(), s));
     h->r = r;
     h->mu = mu;
     return SUN_OK;
@@ -243,8 +247,20 @@ static int sun_wlop_fields_to_host_body(sun_wlop* h, double* out) {
     const int nreal = 2 * lat->d.nc * lat->d.nc;
     const bool f32 = lat->d.precision == SUN_PREC_F32;
     std::vector<float> raw(f32 ? V * nreal : 0);
+    std::vector<double> planes(h->planes() ? h->stride / sizeof(double) : 0);
     for (int k = 0; k < h->nop; k++) {
         double* dst = out + (size_t)k * V * nreal;
+        if (h->planes()) {  // of 16 bytes: real q of site l
+            const size_t per = f32 ? 4 : 2;
+            HIP_TRY(hipMemcpy(planes.data(), (char*)h->ops + (size_t)k * h->stride, h->stride, hipMemcpyDeviceToHost));
+            const float* p32 = (const float*)planes.data();
+            for (size_t q = 0; q < (size_t)nreal; q++)
+                for (size_t l = 0; l < V; l++) {
+                    const size_t at = (q / per * V + l) * per + q % per;
+                    dst[l * nreal + q] = f32 ? p32[at] : planes[at];
+                }
+            continue;
+        }
         if (!f32) {
             HIP_TRY(hipMemcpy(dst, (char*)h->ops + (size_t)k * h->stride, h->stride, hipMemcpyDeviceToHost));
             continue;
