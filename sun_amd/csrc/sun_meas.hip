@@ -171,8 +171,9 @@ WlPlanes wl_planes(const sun_lattice* lat, int tmax) {
     const Geom& g = lat->g;
     const size_t reals = (size_t)2 * lat->d.nc * lat->d.nc;
     WlPlanes w;
-    w.ps[0] = plane_shape(g, tmax + 1, (int)(reals * lat->d.precision));
-    w.ps[1] = plane_shape(g, tmax + 1, (int)(reals * sizeof(double)));
+    const bool f64 = lat->d.precision == SUN_PREC_F64;
+    w.ps[0] = plane_shape(g, tmax + 1, (int)(reals * lat->d.precision), lat->d.nc == 2 || (lat->d.nc == 3 && !f64));
+    w.ps[1] = plane_shape(g, tmax + 1, (int)(reals * sizeof(double)), lat->d.nc == 2);
     w.off = ((size_t)g.str[3] * (g.X[3] + 1) * reals * sizeof(double) + 255) & ~(size_t)255;
     w.lines = w.off + (((size_t)g.V * (reals / 2 + 3) * lat->d.precision + 255) & ~(size_t)255);
     w.per_radius = (size_t)3 * (tmax + 1) * std::max(w.ps[0].blocks, w.ps[1].blocks) * sizeof(double2);
@@ -187,11 +188,41 @@ size_t wl_part_bytes(const sun_lattice* lat, int tmax) {
     return (size_t)3 * (tmax + 1) * monitor_blocks(lat->g) * sizeof(double2);
 }
 
-// Both entry points take the same route, for the same bits: by planes where they fit LDS, except
-// sizes that sun_wilson_loops_noalloc accepts but whose time lines its array does not hold
-bool wl_takes_planes(const sun_lattice* lat, const WlPlanes& w, int tmax) {
-    if (!w.fits()) return false;
-    if (wl_line_bytes(lat) + wl_part_bytes(lat, tmax) > kNoAllocScratchBytes) return true;
+bool wl_fits_noalloc(const sun_lattice* lat, int tmax) {
+    return wl_line_bytes(lat) + wl_part_bytes(lat, tmax) <= kNoAllocScratchBytes;
+}
+
+// Planes cost the time lines, a chain over the lattice's times; multiplied out, every radius and
+// T costs its products.  Estimates of both, us: a launch's latency, and per time, radius, T and
+// 2^20 sites what calls of 4^4 to 32^4 with r <= 8 and T <= 16 take (rows N = 2, 3, 4, FP32 and FP64;
+// fitted to 1458 calls by either route).  The route so chosen takes 0.7 % more than the better
+// one on the average, at most 8 % more than multiplied out before there were planes (SU(3) FP32
+// r, T <= 1: 4^3 x 128 219 us by planes, 52 multiplied out; 24^3 x 32 r = 4, T = 0 366 and 352, r = 8 549
+// and 616; r, T <= 2 at 16^4 102 and 103).
+struct WlCost {
+    double time, site, radius, radius_site, loop_site;       // planes
+    double p_radius, p_loop, p_site, p_loop_site;            // products
+};
+constexpr WlCost kWlCost[3][2] = {
+    {{0.44, 68, 2.7, 33, 2.0, 2.7, 0.9, 63, 18}, {0.51, 82, 2.8, 53, 2.8, 2.8, 1.1, 117, 38}},
+    {{1.2, 153, 4.8, 97, 4.8, 2.7, 1.7, 122, 45}, {1.5, 235, 5.6, 167, 8.5, 3.5, 2.6, 270, 128}},
+    {{2.4, 326, 10, 329, 13, 3.4, 2.8, 257, 106}, {3.0, 398, 18, 649, 45, 2.9, 4.4, 582, 302}}};
+bool wl_planes_faster(const sun_lattice* lat, int rmax, int tmax) {
+    const Geom& g = lat->g;
+    const WlCost& c = kWlCost[lat->d.nc - 2][lat->d.precision == SUN_PREC_F64];
+    const double sites = (double)g.V / (1 << 20);
+    double planes = 56 + c.time * g.X[3] + c.site * sites + rmax * (c.radius + sites * (c.radius_site + c.loop_site * (tmax + 1)));
+    // the launches of sun_wilson_loops_noalloc's other route, which find nothing to do
+    if (wl_fits_noalloc(lat, tmax)) planes += 3.6 * (rmax + 1);
+    return planes < 24 + (rmax + 1) * (c.p_radius + c.p_loop * (tmax + 1) + sites * (c.p_site + c.p_loop_site * tmax));
+}
+
+// Both entry points take the same route, for the same bits: by planes where they fit LDS and are
+// the faster ones, except sizes that sun_wilson_loops_noalloc accepts but whose time lines its
+// array does not hold
+bool wl_takes_planes(const sun_lattice* lat, const WlPlanes& w, int rmax, int tmax) {
+    if (!w.fits() || !wl_planes_faster(lat, rmax, tmax)) return false;
+    if (!wl_fits_noalloc(lat, tmax)) return true;
     return w.lines + w.per_radius <= kNoAllocScratchBytes && line_blocks(lat->g) * sizeof(int) <= kNoAllocStateBytes;
 }
 
@@ -220,16 +251,38 @@ int wl_by_planes(sun_lattice* lat, const WlPlanes& w, int rmax, int tmax, double
     return SUN_OK;
 }
 
-// every product multiplied out; where state is given, only if it is kLinesBad
-int wl_by_products(sun_lattice* lat, int rmax, int tmax, const Field& lines, double2* part, const int* state,
-                   double2* res, hipStream_t s) {
+// Every product multiplied out, in `bytes` bytes at base; where state is given, only if it is
+// kLinesBad.  Two line fields where sun_wilson_loops_noalloc's array holds them (for both entry
+// points: the same bits), so that a radius is one launch and the sums of several radii another.
+bool wl_two_fields(const sun_lattice* lat, int tmax) {
+    return 2 * wl_line_bytes(lat) + wl_part_bytes(lat, tmax) <= kNoAllocScratchBytes;
+}
+size_t wl_products_bytes(const sun_lattice* lat, int rmax, int tmax) {
+    const size_t part = wl_part_bytes(lat, tmax);
+    if (!wl_two_fields(lat, tmax)) return wl_line_bytes(lat) + part;
+    return std::min(2 * wl_line_bytes(lat) + (rmax + 1) * part, kNoAllocScratchBytes);
+}
+int wl_by_products(sun_lattice* lat, int rmax, int tmax, char* base, size_t bytes, const int* state, double2* res,
+                   hipStream_t s) {
     const Geom& g = lat->g;
+    const size_t full = (size_t)2 * lat->d.nc * lat->d.nc * (size_t)lat->d.precision;  // 18-real record
+    const size_t line = wl_line_bytes(lat), part_bytes = wl_part_bytes(lat, tmax);
+    const bool two = wl_two_fields(lat, tmax);
+    const Field lines[2] = {make_field(base, 3 * (size_t)g.V, full), make_field(base + (two ? line : 0), 3 * (size_t)g.V, full)};
+    const size_t at_part = two ? 2 * line : line;
+    double2* part = reinterpret_cast<double2*>(base + at_part);
     const int nb[3] = {0, 0, monitor_blocks(g)};
-    for (int r = 0; r <= rmax; r++) {
-        HIP_TRY(lat->ops->wl_lines(lat->f, lines, g, r, state, s));
-        HIP_TRY(lat->ops->wl_loops(lat->f, lines, g, r, tmax, state, part, s));
-        HIP_TRY(launch_wl_finalize(part, nb, 1, tmax, wl_scale(lat), state, line_blocks(g),
-                                   res + (size_t)r * (tmax + 1), s));
+    const int group = two ? (int)std::min<size_t>((size_t)rmax + 1, (bytes - at_part) / part_bytes) : 1;
+    for (int lo = 0; lo <= rmax; lo += group) {
+        const int hi = std::min(rmax + 1, lo + group);
+        for (int r = lo; r < hi; r++) {
+            double2* p = part + (r - lo) * (part_bytes / sizeof(double2));
+            if (!two) HIP_TRY(lat->ops->wl_lines(lat->f, lines[0], g, r, state, s));
+            HIP_TRY(lat->ops->wl_loops(lat->f, lines[two ? r & 1 : 0], two ? &lines[~r & 1] : nullptr, r == rmax, g, r, tmax,
+                                       state, p, s));
+        }
+        HIP_TRY(launch_wl_finalize(part, nb, hi - lo, tmax, wl_scale(lat), state, line_blocks(g),
+                                   res + (size_t)lo * (tmax + 1), s));
     }
     return SUN_OK;
 }
@@ -248,7 +301,7 @@ static int sun_wilson_loops_body(sun_lattice* lat, int rmax, int tmax, double* o
     std::vector<double2> h(nres);
     const WlPlanes w = wl_planes(lat, tmax);
     bool done = false;
-    if (wl_takes_planes(lat, w, tmax)) {
+    if (wl_takes_planes(lat, w, rmax, tmax)) {
         constexpr size_t kPartBytes = size_t(64) << 20;  // of partial sums at a time
         const size_t part = std::max(w.per_radius, std::min(w.per_radius * (rmax + 1), kPartBytes));
         std::vector<int> st(line_blocks(g));
@@ -264,14 +317,10 @@ static int sun_wilson_loops_body(sun_lattice* lat, int rmax, int tmax, double* o
         done = std::find(st.begin(), st.end(), kLinesBad) == st.end();
     }
     if (!done) {
-        const size_t full = (size_t)2 * lat->d.nc * lat->d.nc * (size_t)lat->d.precision;  // 18-real record
-        const size_t nline = 3 * (size_t)g.V;
-        const size_t at_part = (nline * full + 255) & ~(size_t)255;
-        const size_t at_res = at_part + (size_t)3 * (tmax + 1) * monitor_blocks(g) * sizeof(double2);
+        const size_t at_res = wl_products_bytes(lat, rmax, tmax);
         CallScratch mem(lat->ctx, s);
         HIP_TRY(mem.take(at_res + res_bytes));
-        SUN_TRY(wl_by_products(lat, rmax, tmax, make_field(mem.at(), nline, full), (double2*)mem.at(at_part), nullptr,
-                               (double2*)mem.at(at_res), s));
+        SUN_TRY(wl_by_products(lat, rmax, tmax, mem.at(), at_res, nullptr, (double2*)mem.at(at_res), s));
         HIP_TRY(hipMemcpyAsync(h.data(), mem.at(at_res), nres * sizeof(double2), hipMemcpyDeviceToHost, s));
         HIP_TRY(mem.sync());
     }
@@ -299,8 +348,6 @@ extern "C" int sun_wilson_loops_noalloc(sun_lattice* lat, int rmax, int tmax, do
     if (rmax < 0 || tmax < 0 || rmax > g.X[0] || rmax > g.X[1] || rmax > g.X[2] || tmax > g.X[3])
         return fail(SUN_ERR_INVALID, "sun_wilson_loops_noalloc: rmax %d, tmax %d outside the lattice", rmax, tmax);
     if (!lat->ctx->scratch) return fail(SUN_ERR_STATE, "sun_wilson_loops_noalloc: no scratch array on this device");
-    const size_t full = (size_t)2 * lat->d.nc * lat->d.nc * (size_t)lat->d.precision;  // 18-real record
-    const size_t nline = 3 * (size_t)g.V;
     const size_t line_bytes = wl_line_bytes(lat), part_bytes = wl_part_bytes(lat, tmax);
     if (line_bytes + part_bytes > kNoAllocScratchBytes)
         return fail(SUN_ERR_BUDGET,
@@ -313,11 +360,10 @@ extern "C" int sun_wilson_loops_noalloc(sun_lattice* lat, int rmax, int tmax, do
     double2* res = reinterpret_cast<double2*>(dev_out);
     const WlPlanes w = wl_planes(lat, tmax);
     int* state = nullptr;
-    if (wl_takes_planes(lat, w, tmax)) {
+    if (wl_takes_planes(lat, w, rmax, tmax)) {
         state = reinterpret_cast<int*>(base + kNoAllocScratchBytes);
         SUN_TRY(wl_by_planes(lat, w, rmax, tmax, reinterpret_cast<double*>(base),
                              reinterpret_cast<double2*>(base + w.lines), kNoAllocScratchBytes - w.lines, state, res, s));
     }
-    return wl_by_products(lat, rmax, tmax, make_field(base, nline, full), reinterpret_cast<double2*>(base + line_bytes),
-                          state, res, s);
+    return wl_by_products(lat, rmax, tmax, reinterpret_cast<char*>(base), kNoAllocScratchBytes, state, res, s);
 }

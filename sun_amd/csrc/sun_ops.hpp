@@ -140,7 +140,7 @@ struct PlaneShape {
     int sums, lds;  // bytes before the sums, and in all
 };
 // the shape for matrices of `bytes` bytes, or sites = 0 where the times do not fit
-inline PlaneShape plane_shape(const Geom& g, int T1, int bytes) {
+inline PlaneShape plane_shape(const Geom& g, int T1, int bytes, bool two_wgs) {
     constexpr int kThreads = 256, kLds = 156 * 1024;
     PlaneShape p{};
     // chunks of 5, 7 or 9 T (compiled kernels), as few as possible, then as small as possible
@@ -149,11 +149,12 @@ inline PlaneShape plane_shape(const Geom& g, int T1, int bytes) {
     p.extent = g.X[3] + (n * p.chunk + 1) / 2 * 2;
     const long long sums = 8ll * kThreads / 64 * 2 * T1;
     const long long most = (kLds - sums) / ((long long)p.extent * bytes);
-    // two workgroups a CU where they fit
+    // two workgroups a CU where they fit and registers allow two (FP64 SU(4), which they do not: half of
+    // the threads were without a site; SU(3) 13 sites for 16)
     const long long two = (kLds / 2 - sums) / ((long long)p.extent * bytes);
     long long sites = 2 * kThreads / g.X[3];
     if (sites > most) sites = most;
-    if (two >= 1 && two < sites) sites = two;
+    if (two_wgs && two >= 1 && two < sites) sites = two;
     if (sites < 1 || g.X[3] > 2 * kThreads) return p;
     p.sites = (int)sites;
     p.blocks = (g.str[3] + p.sites - 1) / p.sites;
@@ -221,11 +222,12 @@ struct OpsTable {
     // lines are near to unitary, ps[1] where not; nothing where they are kLinesBad
     hipError_t (*wl_plane)(const Field& f, const Geom&, int r_lo, int r_hi, int T1, int next, const double* P,
                            const void* E, const int* state, const PlaneShape ps[2], double2* partials, hipStream_t);
-    // the same with the links multiplied out: the Wilson lines of radius r, then its loops;
+    // the same with the links multiplied out: the Wilson lines of radius r, then its loops, or, with
+    // a second field `next`, the loops and there the lines of r + 1 (none after the last radius);
     // where state is given, only if it is kLinesBad
     hipError_t (*wl_lines)(const Field& f, const Field& lines, const Geom&, int r, const int* state, hipStream_t);
-    hipError_t (*wl_loops)(const Field& f, const Field& lines, const Geom&, int r, int tmax, const int* state,
-                           double2* partials, hipStream_t);
+    hipError_t (*wl_loops)(const Field& f, const Field& lines, const Field* next, bool last, const Geom&, int r, int tmax,
+                           const int* state, double2* partials, hipStream_t);
     // operator-basis Wilson loops: the operator fields of direction mu at radius r
     // (family 0: 10 slots, 1: 25; slot k, V matrices of 2 N^2 reals one after another or, where
     // `planes`, like the links, at ops + k * stride; rt8 = 2 sqrt 2).  exact: FP64 fields with the reference's products one
