@@ -25,11 +25,18 @@ namespace {
 // two, 120939 / 118666 for 32).
 constexpr int kGraphIters = 24;
 
+// A call's graph.  Its executable form goes only when its launches are done: it holds their
+// kernel arguments.
 struct GraphGuard {
+    hipStream_t s;
     hipGraph_t g = nullptr;
     hipGraphExec_t x = nullptr;
+    explicit GraphGuard(hipStream_t s) : s(s) {}
     ~GraphGuard() {
-        if (x) hipGraphExecDestroy(x);
+        if (x) {
+            hipStreamSynchronize(s);
+            hipGraphExecDestroy(x);
+        }
         if (g) hipGraphDestroy(g);
     }
 };
@@ -100,8 +107,8 @@ static int sun_generate_body(sun_lattice* lat, const sun_generate_desc* d, void*
     HIP_TRY(hipMemcpyAsync(lat->sweep_dev, &first, sizeof(uint32_t), hipMemcpyHostToDevice, s));
     HIP_TRY(hipStreamSynchronize(s));
 
+    GraphGuard plain(s), with_reunit(s);  // after the wait at the end
     if (d->use_graph && d->n_iter >= kGraphIters) {
-        GraphGuard plain, with_reunit;
         const bool need_plain = d->reunit_every != 1;
         const bool need_reunit = d->reunit_every >= 1;
         if (need_plain)
@@ -458,8 +465,8 @@ static int sun_batch_generate_body(sun_batch* b, uint32_t first_sweep, int n_ite
     const uint32_t zero = 0;
     HIP_TRY(hipMemcpyAsync(b->iter_dev, &zero, sizeof(uint32_t), hipMemcpyHostToDevice, s));
     HIP_TRY(hipStreamSynchronize(s));
+    GraphGuard plain(s), with_reunit(s);  // after the wait at the end
     if (use_graph && n_iter >= kGraphIters) {
-        GraphGuard plain, with_reunit;
         if (reunit_every != 1) SUN_TRY(capture(s, plain, [&] { return batch_iteration(b, n_or, false, measure, s); }));
         if (reunit_every >= 1)
             SUN_TRY(capture(s, with_reunit, [&] { return batch_iteration(b, n_or, true, measure, s); }));

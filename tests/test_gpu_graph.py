@@ -86,3 +86,19 @@ def test_chunks_on_several_streams_replay_a_graph(ctx, nc, storage, prec, count)
             lat.close()
     assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
     assert np.array_equal(out[0][2], out[1][2]) and np.array_equal(out[0][3], out[1][3])
+
+
+def test_many_chunks_in_flight_at_the_end_of_a_call(ctx):
+    """Eleven chunks and iterations of 10 ms: a call has launched all its replays long before the first is done,
+    and keeps their graph until the last is."""
+    lats = [sun_amd.Lattice(ctx, 3, (16,) * 4, 5.9, 18, 8) for _ in range(24)]
+    batch = sun_amd.Batch(ctx, lats, range(24))
+    rows = []
+    for graph in (False, True):
+        for i, lat in enumerate(lats):
+            lat.hot_start(i)
+        rows.append([batch.generate(0, 24, n_or=3, use_graph=graph), batch.generate(24, 40, n_or=3, use_graph=graph)])
+    assert all(np.array_equal(a, b) for a, b in zip(*rows))
+    batch.close()
+    for lat in lats:
+        lat.close()
