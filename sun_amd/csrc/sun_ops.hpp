@@ -231,7 +231,7 @@ struct OpsTable {
     // operator-basis Wilson loops: the operator fields of direction mu at radius r
     // (family 0: 10 slots, 1: 25; slot k, V matrices of 2 N^2 reals one after another or, where
     // `planes`, like the links, at ops + k * stride; rt8 = 2 sqrt 2).  exact: FP64 fields with the reference's products one
-    // by one, otherwise from shared products (33: in kWlopAuxSlots more slots at aux; A0: slot
+    // by one (33 also where aux is null), otherwise from shared products (33: in kWlopAuxSlots more slots at aux; A0: slot
     // 9 is left as it is)
     hipError_t (*wlop_fields)(const Field& f, char* ops, char* aux, size_t stride, const Geom&, int family, int r,
                               int mu, double rt8, bool exact, bool planes, hipStream_t);

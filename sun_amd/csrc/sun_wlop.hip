@@ -24,10 +24,10 @@ struct sun_wlop {
     size_t stride = 0;      // bytes of one slot (V entries)
     size_t held = 0;        // bytes of the block that all the following lie in
     void* ops = nullptr;    // nop slots
-    void* aux = nullptr;    // scratch slots of the 33 family
+    void* aux = nullptr;    // scratch slots of the 33 family's shared products, or none
     double* partials = nullptr;
     int nb = 0, rows = 0;   // workgroups of the fallback and of the matrix-core correlator
-    bool direct = false;    // few T: without time lines
+    bool direct = false;    // few T, or no memory for them: without time lines
     bool planes() const { return wlop_planes(direct, lat->d.nc, lat->d.precision == SUN_PREC_F64, nop); }
     double* lines = nullptr;   // time lines: X3 + tmax times of every spatial site
     double* inverses = nullptr;  // their inverses, X3 times
@@ -77,7 +77,8 @@ int check_radius(const sun_wlop* h, int r, int mu, const char* what) {
 
 }  // namespace
 
-extern "C" int sun_wlop_create(sun_lattice* lat, int family, int tmax, sun_wlop** out) {
+// shared: the fields will come from shared products (fields())
+static int create(sun_lattice* lat, int family, int tmax, bool shared, sun_wlop** out) {
     if (!out) return fail(SUN_ERR_INVALID, "sun_wlop_create: NULL handle pointer");
     *out = nullptr;
     if (!lat) return fail(SUN_ERR_INVALID, "sun_wlop_create: NULL lattice");
@@ -98,35 +99,51 @@ extern "C" int sun_wlop_create(sun_lattice* lat, int family, int tmax, sun_wlop*
     h->nb = monitor_blocks(g);
     h->rows = wlop_corr_blocks(g);
     h->direct = wlop_direct(nop, tmax + 1, lat);
+    // scratch slots for the 33 family's shared products, which FP64 fields that are handed out are not
+    bool aux = family == SUN_WLOP_33 && (shared || lat->d.precision == SUN_PREC_F32);
     const size_t nout = (size_t)nop * nop * (tmax + 1);
     const size_t npart = nout * (size_t)std::max(h->nb, h->rows);
     const size_t line = (size_t)2 * lat->d.nc * lat->d.nc * sizeof(double), vs = (size_t)g.str[3];
-    size_t total = 0;
-    auto part = [&](size_t bytes) {
-        const size_t at = total;
-        total += (bytes + 255) & ~(size_t)255;
-        return at;
+    // the parts of a block: without one counted, then with it
+    auto lay_out = [&](char* base) {
+        size_t total = 0;
+        auto part = [&](size_t bytes) {
+            char* p = base + total;
+            total += (bytes + 255) & ~(size_t)255;
+            return p;
+        };
+        part((size_t)nop * h->stride);
+        h->partials = (double*)part(npart * sizeof(double));
+        h->acc = (double*)part(nout * sizeof(double));
+        h->aux = aux ? part((size_t)kWlopAuxSlots * h->stride) : nullptr;
+        if (!h->direct) {
+            h->lines = (double*)part(vs * (g.X[3] + tmax) * line);
+            h->inverses = (double*)part(vs * g.X[3] * line);
+            h->state = (int*)part(line_blocks(g) * sizeof(int));
+        }
+        return total;
     };
-    part((size_t)nop * h->stride);
-    const size_t at_aux = part(family == SUN_WLOP_33 ? (size_t)kWlopAuxSlots * h->stride : 0);
-    const size_t at_partials = part(npart * sizeof(double)), at_lines = part(vs * (g.X[3] + tmax) * line);
-    const size_t at_inverses = part(vs * g.X[3] * line), at_state = part(line_blocks(g) * sizeof(int));
-    const size_t at_acc = part(nout * sizeof(double));
-    HIP_TRY_CLEANUP(lat->ctx->spare.take(total, &h->ops, &h->held), release(h));
+    hipError_t e = lat->ctx->spare.take(lay_out(nullptr), &h->ops, &h->held);
+    if (e == hipErrorOutOfMemory && (aux || !h->direct)) {
+        // the operators and sums alone: the fields multiplied out path by path, the correlators link by link
+        hipGetLastError();
+        aux = false;
+        h->direct = true;
+        e = lat->ctx->spare.take(lay_out(nullptr), &h->ops, &h->held);
+    }
+    HIP_TRY_CLEANUP(e, release(h));
     char* base = static_cast<char*>(h->ops);
-    if (family == SUN_WLOP_33)
-        h->aux = base + at_aux;
-    else  // slot 9 of A0 is zero throughout
+    lay_out(base);
+    if (family == SUN_WLOP_A0)  // slot 9 is zero throughout
         HIP_TRY_CLEANUP(hipMemset(base + 9 * h->stride, 0, h->stride), release(h));
-    h->partials = (double*)(base + at_partials);
-    h->lines = (double*)(base + at_lines);
-    h->inverses = (double*)(base + at_inverses);
-    h->state = (int*)(base + at_state);
-    h->acc = (double*)(base + at_acc);
     HIP_TRY_CLEANUP(hipMemset(h->acc, 0, nout * sizeof(double)), release(h));
     HIP_TRY_CLEANUP(hipStreamSynchronize(nullptr), release(h));  // the handle's streams do not wait for it
     *out = h;
     return SUN_OK;
+}
+
+extern "C" int sun_wlop_create(sun_lattice* lat, int family, int tmax, sun_wlop** out) {
+    return create(lat, family, tmax, false, out);
 }
 
 extern "C" int sun_wlop_destroy(sun_wlop* h) {
@@ -283,7 +300,7 @@ static int sun_wilson_loops_ops_body(sun_lattice* lat, int family, int rmax, int
     if (rmax < 2 || rmax > g.X[0] || rmax > g.X[1] || rmax > g.X[2])
         return fail(SUN_ERR_INVALID, "sun_wilson_loops_ops: rmax %d outside 2..(smallest spatial extent)", rmax);
     sun_wlop* h = nullptr;
-    SUN_TRY(sun_wlop_create(lat, family, tmax, &h));
+    SUN_TRY(create(lat, family, tmax, true, &h));
     const size_t n = (size_t)h->nop * h->nop * (tmax + 1);
     const double norm = (double)g.V * 3.0 * lat->d.nc;  // test.cpp:290
     const hipStream_t s = pick_stream(lat, stream);
