@@ -129,6 +129,9 @@ hipError_t sun::Workspaces::allocate(void** p, size_t bytes) {
 }
 
 hipError_t sun::CallScratch::take(size_t bytes) {
+    // a block belongs to its context's device, whatever the caller's current one is
+    const hipError_t e = hipSetDevice(ctx_->device);
+    if (e != hipSuccess) return e;
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(s_, &st) != hipSuccess || st != hipStreamCaptureStatusNone) {
         hipGetLastError();
