@@ -68,7 +68,9 @@ typedef struct {
 /* ---- runtime ----------------------------------------------------------------- */
 /* initCULQCD(gpuid, verbosity, tune)            include/comm_mpi.h:43, comm_mpi.cpp:92-184 */
 int sun_init(int device, int verbosity, int tune, sun_ctx **out);
-/* EndCULQCD(status) without exit()               include/comm_mpi.h:45, comm_mpi.cpp:186-210 */
+/* EndCULQCD(status) without exit()               include/comm_mpi.h:45, comm_mpi.cpp:186-210.
+ * Measurements and host exchange keep up to 2 GiB of their device scratch with the context
+ * between calls; it is given back here, and whenever an allocation of the context fails. */
 int sun_finalize(sun_ctx *ctx);
 /* errorCULQCD message                            include/comm_mpi.h:116-120 */
 const char *sun_last_error(void);

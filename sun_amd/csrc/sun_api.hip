@@ -294,9 +294,9 @@ int sun::lattice_alloc(sun_ctx* ctx, const sun_lattice_desc* d, sun_lattice** ou
     (void)tail;
     set_planes(L);
     L->npart = partial_slots(L->g);
-    e = hipMalloc(&L->partials, sizeof(double2) * (size_t)L->npart);
-    if (e == hipSuccess) e = hipMalloc(&L->dres, sizeof(double2) * kResSlots);
-    if (e == hipSuccess) e = hipMalloc(&L->sweep_dev, sizeof(uint32_t));
+    e = ctx->spare.allocate((void**)&L->partials, sizeof(double2) * (size_t)L->npart);
+    if (e == hipSuccess) e = ctx->spare.allocate((void**)&L->dres, sizeof(double2) * kResSlots);
+    if (e == hipSuccess) e = ctx->spare.allocate((void**)&L->sweep_dev, sizeof(uint32_t));
     if (e == hipSuccess) e = hipHostMalloc(&L->hres, sizeof(double2) * kResSlots, hipHostMallocDefault);
     if (e != hipSuccess) {
         hipGetLastError();

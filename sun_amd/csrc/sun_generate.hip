@@ -41,12 +41,12 @@ struct GraphGuard {
     }
 };
 
-int ensure_obs(double2** buf, int* cap, int n) {
+int ensure_obs(sun_ctx* ctx, double2** buf, int* cap, int n) {
     if (*cap >= n) return SUN_OK;
     if (*buf) hipFree(*buf);
     *buf = nullptr;
     *cap = 0;
-    HIP_TRY(hipMalloc(buf, sizeof(double2) * (size_t)n));
+    HIP_TRY(ctx->spare.allocate((void**)buf, sizeof(double2) * (size_t)n));
     *cap = n;
     return SUN_OK;
 }
@@ -101,7 +101,7 @@ static int sun_generate_body(sun_lattice* lat, const sun_generate_desc* d, void*
     if (d->n_iter == 0) return SUN_OK;
     hipStream_t s = pick_stream(lat, stream);
     const bool measure = d->measure != 0;
-    if (measure) SUN_TRY(ensure_obs(&lat->obs_dev, &lat->obs_cap, 2 * d->n_iter));
+    if (measure) SUN_TRY(ensure_obs(lat->ctx, &lat->obs_dev, &lat->obs_cap, 2 * d->n_iter));
     const uint32_t first = d->first_sweep;
     SUN_TRY(tune_lattice(lat, s));
     HIP_TRY(hipMemcpyAsync(lat->sweep_dev, &first, sizeof(uint32_t), hipMemcpyHostToDevice, s));
@@ -227,12 +227,12 @@ static void build_schedule(sun_batch::Schedule& sc, sun_lattice* const* lats, in
     sc.h_update = tu;
 }
 
-static hipError_t upload_schedule(sun_batch::Schedule& sc, const std::vector<BatchEntry>& tr,
+static hipError_t upload_schedule(sun_ctx* ctx, sun_batch::Schedule& sc, const std::vector<BatchEntry>& tr,
                                   const std::vector<BatchEntry>& tp) {
     const size_t bytes = sizeof(BatchEntry) * sc.h_update.size();
-    hipError_t e = hipMalloc(&sc.t_update, bytes);
-    if (e == hipSuccess) e = hipMalloc(&sc.t_reunit, bytes);
-    if (e == hipSuccess) e = hipMalloc(&sc.t_plaq, bytes);
+    hipError_t e = ctx->spare.allocate((void**)&sc.t_update, bytes);
+    if (e == hipSuccess) e = ctx->spare.allocate((void**)&sc.t_reunit, bytes);
+    if (e == hipSuccess) e = ctx->spare.allocate((void**)&sc.t_plaq, bytes);
     if (e == hipSuccess) e = hipMemcpy(sc.t_update, sc.h_update.data(), bytes, hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(sc.t_reunit, tr.data(), bytes, hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(sc.t_plaq, tp.data(), bytes, hipMemcpyHostToDevice);
@@ -283,14 +283,14 @@ static int sun_batch_create_body(sun_ctx* ctx, int n, sun_lattice* const* lats, 
     build_schedule(b->gen, lats, n, seeds, kBatchChunkBytes, kBatchBranches, tr_gen, tp_gen);
     build_schedule(b->step, lats, n, seeds, kCacheChunkBytes, 1, tr_step, tp_step);
     hipError_t e = hipSetDevice(ctx->device);
-    if (e == hipSuccess) e = hipMalloc(&b->partials, sizeof(double2) * (size_t)cp_all);
-    if (e == hipSuccess) e = hipMalloc(&b->d_out, sizeof(double2) * n);
+    if (e == hipSuccess) e = ctx->spare.allocate((void**)&b->partials, sizeof(double2) * (size_t)cp_all);
+    if (e == hipSuccess) e = ctx->spare.allocate((void**)&b->d_out, sizeof(double2) * n);
     if (e == hipSuccess)
         for (int i = 0; i < n; i++) tp_gen[i].partials = tp_step[i].partials = b->partials + poff[i];
-    if (e == hipSuccess) e = hipMalloc(&b->iter_dev, sizeof(uint32_t));
+    if (e == hipSuccess) e = ctx->spare.allocate((void**)&b->iter_dev, sizeof(uint32_t));
     if (e == hipSuccess) e = hipHostMalloc(&b->h_out, sizeof(double2) * n, hipHostMallocDefault);
-    if (e == hipSuccess) e = upload_schedule(b->gen, tr_gen, tp_gen);
-    if (e == hipSuccess) e = upload_schedule(b->step, tr_step, tp_step);
+    if (e == hipSuccess) e = upload_schedule(ctx, b->gen, tr_gen, tp_gen);
+    if (e == hipSuccess) e = upload_schedule(ctx, b->step, tr_step, tp_step);
     if (e == hipSuccess) e = hipEventCreateWithFlags(&b->fork, hipEventDisableTiming);
     for (int k = 1; k < kBatchBranches && e == hipSuccess; k++) {
         e = hipStreamCreateWithFlags(&b->branch[k], hipStreamNonBlocking);
@@ -460,7 +460,7 @@ static int sun_batch_generate_body(sun_batch* b, uint32_t first_sweep, int n_ite
     hipStream_t s = batch_stream(b, stream);
     const int n = (int)b->lats.size();
     const bool measure = obs != nullptr;
-    if (measure) SUN_TRY(ensure_obs(&b->obs_dev, &b->obs_cap, n * n_iter));
+    if (measure) SUN_TRY(ensure_obs(b->ctx, &b->obs_dev, &b->obs_cap, n * n_iter));
     SUN_TRY(batch_set_sweeps(b, b->gen, nullptr, first_sweep, s));
     const uint32_t zero = 0;
     HIP_TRY(hipMemcpyAsync(b->iter_dev, &zero, sizeof(uint32_t), hipMemcpyHostToDevice, s));

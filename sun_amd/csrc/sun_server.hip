@@ -197,12 +197,12 @@ int make_group(sun_server* S, const sun_lattice* L, int n_or, int reunit, Group*
     const size_t tb = sizeof(BatchEntry) * (size_t)g->cap;
     hipError_t e = hipStreamCreateWithFlags(&g->stream, hipStreamNonBlocking);
     if (e == hipSuccess) e = hipEventCreateWithFlags(&g->done, hipEventDisableTiming);
-    if (e == hipSuccess) e = hipMalloc(&g->t_update, tb);
-    if (e == hipSuccess) e = hipMalloc(&g->t_reunit, tb);
-    if (e == hipSuccess) e = hipMalloc(&g->t_plaq, tb);
-    if (e == hipSuccess) e = hipMalloc(&g->t_poly, tb);
-    if (e == hipSuccess) e = hipMalloc(&g->d_plaq, sizeof(double2) * (size_t)g->cap);
-    if (e == hipSuccess) e = hipMalloc(&g->d_poly, sizeof(double2) * (size_t)g->cap);
+    if (e == hipSuccess) e = S->ctx->spare.allocate((void**)&g->t_update, tb);
+    if (e == hipSuccess) e = S->ctx->spare.allocate((void**)&g->t_reunit, tb);
+    if (e == hipSuccess) e = S->ctx->spare.allocate((void**)&g->t_plaq, tb);
+    if (e == hipSuccess) e = S->ctx->spare.allocate((void**)&g->t_poly, tb);
+    if (e == hipSuccess) e = S->ctx->spare.allocate((void**)&g->d_plaq, sizeof(double2) * (size_t)g->cap);
+    if (e == hipSuccess) e = S->ctx->spare.allocate((void**)&g->d_poly, sizeof(double2) * (size_t)g->cap);
     if (e != hipSuccess) {
         hipGetLastError();
         free_group(g);
