@@ -259,15 +259,18 @@ struct OpsTable {
 //   FP32 at 20^4: 9.3 / 8.1; 8-real FP32 at 28^4: 30.4 / 28.0), except the 8-real heatbath of
 //   large lattices (48^4: 252 / more than 260).
 // - Up to 2^18 sites the chip is not full: one wavefront per workgroup spreads over more
-//   CUs (FP64 SU(3) at 8^4: 13.7 / 10.7, at 12^4: 14.3 / 11.0; at 2^18 sites no difference).
+//   CUs (FP64 SU(3) at 16^3 x 18: 17.7 / 16.0, at 20^4: 32.0 / 29.0, SU(4) FP32 at 8^4: 15.1 /
+//   13.5; at 2^18 sites no difference).
 // - Above, bricks of 16 rows (8 from X0 = 48 on), two apart in x1 and x3, keep the links that
 //   neighbours share in the L2, with no more than two workgroups a CU (FP64 SU(3) at
 //   24^3 x 48: 120 / 104, SU(4) FP32 at 32^4: 169 / 150, FP32 12-real at 32^4: 52.6 / 38.7;
 //   no gain at 2^18 sites, nor below 2^19 for 32-byte links).  Where no brick tiles, linear
 //   (40 x 32^3, 28^4: no shape is faster).
 // - Decoding FP64 links is arithmetic: linear, one wavefront per workgroup (12-real heatbath
-//   at 48^4: 989 / 903), but bricks for 12-real overrelaxation where rows are 16 or 32 sites
-//   (32^4: 167 / 151).
+//   at 48^4: 989 / 903), but bricks for 12-real overrelaxation where they are workgroups of 256,
+//   which rows of 16 and 32 sites make (32^4: 162 / 153, 64 x 32^3: 337 / 307; the 192 threads of
+//   rows of 12 or 24 sites are slower than linear, 24 x 32^3 129 / 116, 48 x 32^3 269 / 241, the 128
+//   of 8 sites no faster).
 inline LaunchCfg default_launch(const OpsTable* ops, const Geom& g, int kernel) {
     LaunchCfg c;
     const bool f64 = ops->real_bytes == 8, full = ops->storage == 18, hb = kernel == 0;
@@ -277,12 +280,12 @@ inline LaunchCfg default_launch(const OpsTable* ops, const Geom& g, int kernel) 
     if (ops->has_piped && (ops->storage == 12 || !hb || g.V <= (1 << 19))) c.piped = 2;
     if (!large || (f64 && !full) || (ops->storage == 8 && c.piped)) c.block = 64;
     bool brick = large && ops->storage != 8;
-    if (f64 && !full) brick = brick && !hb && (rows == 16 || rows == 32);
+    if (f64 && !full) brick = brick && !hb;
     if (full && ops->nc == 2 && !f64) brick = brick && g.V >= (1 << 19);
     if (!brick) return c;
     const int b1 = rows <= 16 ? 2 : 1;
     const int block = brick_block(g, b1, 0, 2, 256);
-    if (!block) return c;
+    if (!block || (f64 && !full && block != 256)) return c;
     c.b1 = b1;
     c.b2 = 0;
     c.b3 = 2;

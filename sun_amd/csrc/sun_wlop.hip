@@ -56,7 +56,7 @@ void release(sun_wlop* h) {
 //   A0 FP64   SU(3) 8^3 x 16 61 / 64 for seven T, 69 / 64 for eight; 12^4 92 / 90 for seven; 16^3 x
 //             32 264 / 306 for four, 330 / 310 for five; 24^3 x 32 698 / 890 for three, 987 / 889
 //             for four; SU(4) 12^3 x 24 211 / 253 for four, 264 / 254 for five
-//   A0 FP32   16^4 140 / 143 for seven, 158 / 142 for eight (8^3 x 16 72 / 76, 16^3 x 32 279 / 240)
+//   A0 FP32   16^4 140 / 143 for seven, 158 / 142 for eight (16^3 x 32 279 / 275, 8^3 x 16 69 / 76)
 //   33 FP64   16^3 x 32 530 / 619 for two, 795 / 642 for three; 24^3 x 32 1742 / 1820 for two
 //   33 FP32   16^3 x 32 593 / 665 for five, 710 / 665 for six; 24^3 x 32 2230 / 2052 for five; SU(4) 770 / 963 for two, 1150 / 964
 //             for three
@@ -65,7 +65,7 @@ bool wlop_direct(int nop, int T1, const sun_lattice* lat) {
     const int V = lat->g.V;
     if (nop > 16) return T1 <= (f64 || lat->d.nc > 3 ? 2 : V > (1 << 18) ? 4 : 5);
     if (f64) return T1 <= (V > (1 << 18) ? 3 : V > 25000 ? 4 : V > 10000 ? 6 : 7);
-    return T1 <= 7;
+    return T1 <= (V <= 10000 ? 8 : 7);
 }
 
 int check_radius(const sun_wlop* h, int r, int mu, const char* what) {
