@@ -88,10 +88,10 @@ namespace sun {
 // Device memory for the length of a call (or of an operator handle): blocks that were given back
 // wait here for the next call.  hipMalloc and hipFree of a measurement's scratch cost 0.1 to 1.5 ms
 // a call, and a wait for memory freed just before; HYP smearing and Wilson loops of 16^3 x 32 SU(3)
-// FP64 (0.5 GB) took 3.8 to 15 ms with them and take 2.2 without.  At most kKeep bytes stay idle (a call that needs
-// more works for longer than the allocation takes), and all of them go back when an allocation of
-// the context fails and at sun_finalize.  A block is given back when the work on it is done, so
-// the next taker may use it on any stream.
+// FP64 (0.5 GB) took 3.8 to 15 ms with them and take 2.2 without.  At most kKeep bytes stay idle
+// (a call that needs more works for longer than the allocation takes), and all of them go back
+// when an allocation of the context fails and at sun_finalize.  A block is given back when the
+// work on it is done, so the next taker may use it on any stream.
 class Workspaces {
 public:
     static constexpr size_t kKeep = size_t(2) << 30;

@@ -211,10 +211,12 @@ bool wl_planes_faster(const sun_lattice* lat, int rmax, int tmax) {
     const Geom& g = lat->g;
     const WlCost& c = kWlCost[lat->d.nc - 2][lat->d.precision == SUN_PREC_F64];
     const double sites = (double)g.V / (1 << 20);
-    double planes = 56 + c.time * g.X[3] + c.site * sites + rmax * (c.radius + sites * (c.radius_site + c.loop_site * (tmax + 1)));
+    double planes = 56 + c.time * g.X[3] + c.site * sites;
+    planes += rmax * (c.radius + sites * (c.radius_site + c.loop_site * (tmax + 1)));
     // the launches of sun_wilson_loops_noalloc's other route, which find nothing to do
     if (wl_fits_noalloc(lat, tmax)) planes += 3.6 * (rmax + 1);
-    return planes < 24 + (rmax + 1) * (c.p_radius + c.p_loop * (tmax + 1) + sites * (c.p_site + c.p_loop_site * tmax));
+    const double radius = c.p_radius + c.p_loop * (tmax + 1) + sites * (c.p_site + c.p_loop_site * tmax);
+    return planes < 24 + (rmax + 1) * radius;
 }
 
 // Both entry points take the same route, for the same bits: by planes where they fit LDS and are
@@ -268,7 +270,8 @@ int wl_by_products(sun_lattice* lat, int rmax, int tmax, char* base, size_t byte
     const size_t full = (size_t)2 * lat->d.nc * lat->d.nc * (size_t)lat->d.precision;  // 18-real record
     const size_t line = wl_line_bytes(lat), part_bytes = wl_part_bytes(lat, tmax);
     const bool two = wl_two_fields(lat, tmax);
-    const Field lines[2] = {make_field(base, 3 * (size_t)g.V, full), make_field(base + (two ? line : 0), 3 * (size_t)g.V, full)};
+    const size_t sites = 3 * (size_t)g.V;
+    const Field lines[2] = {make_field(base, sites, full), make_field(base + (two ? line : 0), sites, full)};
     const size_t at_part = two ? 2 * line : line;
     double2* part = reinterpret_cast<double2*>(base + at_part);
     const int nb[3] = {0, 0, monitor_blocks(g)};

@@ -58,8 +58,8 @@ void release(sun_wlop* h) {
 //             for four; SU(4) 12^3 x 24 211 / 253 for four, 264 / 254 for five
 //   A0 FP32   16^4 140 / 143 for seven, 158 / 142 for eight (16^3 x 32 279 / 275, 8^3 x 16 69 / 76)
 //   33 FP64   16^3 x 32 530 / 619 for two, 795 / 642 for three; 24^3 x 32 1742 / 1820 for two
-//   33 FP32   16^3 x 32 593 / 665 for five, 710 / 665 for six; 24^3 x 32 2230 / 2052 for five; SU(4) 770 / 963 for two, 1150 / 964
-//             for three
+//   33 FP32   16^3 x 32 593 / 665 for five, 710 / 665 for six; 24^3 x 32 2230 / 2052 for five; SU(4) 770 /
+//             963 for two, 1150 / 964 for three
 bool wlop_direct(int nop, int T1, const sun_lattice* lat) {
     const bool f64 = lat->d.precision == SUN_PREC_F64;
     const int V = lat->g.V;
@@ -183,7 +183,9 @@ constexpr LineLimits kLines[2] = {{1.2, 1e8}, {2.0, 1e60}};
 // the time lines of the lattice's present temporal links
 static int time_lines(sun_wlop* h, hipStream_t s) {
     if (h->direct) return SUN_OK;
-    HIP_TRY(h->lat->ops->time_lines(h->lat->f, h->lat->g, h->lat->g.X[3] + h->tmax, false, kLines[h->lat->d.precision == SUN_PREC_F64], h->lines, h->inverses, h->state, s));
+    const sun_lattice* lat = h->lat;
+    HIP_TRY(lat->ops->time_lines(lat->f, lat->g, lat->g.X[3] + h->tmax, false,
+                                 kLines[lat->d.precision == SUN_PREC_F64], h->lines, h->inverses, h->state, s));
     return SUN_OK;
 }
 
